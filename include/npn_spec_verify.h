@@ -159,6 +159,18 @@ int npn_gqa_tail(const float* query, const float* gate, const float* q_norm, con
                  const float* sin, const float* cached_k, const float* cached_v,
                  const float* mask, float* out, int B, int q_heads, int S, void* stream);
 
+/* Workspace bytes for npn_gqa_tail_split with these sizes (0: unsupported sizes). */
+size_t npn_gqa_tail_workspace_size(int B, int q_heads, int S);
+
+/* The same with each sequence's keys split over workgroups, so that small batches use the
+ * whole chip (npn_gqa_tail, which takes no workspace, runs one workgroup per sequence): the
+ * splits' partial softmax results go through the workspace and a second launch merges them.
+ * The sums are associated per split, so the two agree to fp32 rounding, not bitwise. */
+int npn_gqa_tail_split(const float* query, const float* gate, const float* q_norm,
+                       const float* cos, const float* sin, const float* cached_k,
+                       const float* cached_v, const float* mask, float* out, int B, int q_heads,
+                       int S, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Workspace bytes for npn_gqa_tail_verify with these sizes. */
 size_t npn_gqa_tail_verify_workspace_size(int B, int T, int q_heads, int kv_heads, int s_max);
 

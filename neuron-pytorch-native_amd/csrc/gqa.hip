@@ -756,95 +756,314 @@ __global__ __launch_bounds__(256) void gqa_merge_rows_kernel(MergeArgs a) {
 
 // ---------------------------------------------------------------------------------------
 // Decode tail of the reference op (fp32 cache, one kv head, mask shared over the batch).
-// One 256-thread block per sequence b handles its Hq rows; keys in blocks of 64, online
-// softmax in fp32. Wave w scores keys w, w+4, ...: lane l holds dims 4l..4l+3.
+// HBM-bound: every fp32 K and V row is read once for Hq query rows. One workgroup per sequence
+// (the first form of this kernel) left all but B CUs idle and took 3.9 ms at B = 8, Hq = 6,
+// S = 4096 (67 MB, 17 GB/s), so each sequence's keys are split over workgroups, whose
+// (m, l, O) partials a second launch merges.
+// Products run on the fp32 matrix instruction (16x16x4, fp32 operands and sums), heads padded
+// to its 16 columns, which needs no LDS and no cross-lane sums in the loop: the contraction
+// index of each product may be permuted freely as long as both operands agree, so
+//   S^T[16 keys x 16 heads] = K Q'^T: lane (i, g) (i = lane & 15, g = lane >> 4) takes key i,
+//     dims 16 s + 4 g + j at step 4 s + j: a 16-byte load of K feeds four steps;
+//   O[16 heads x 256] += P V: step r takes keys 4 g + r, so lane (i, g)'s S^T register r is its
+//     A operand as it stands, and column i of output tile (n, j) is dim 64 n + 4 i + j, so a
+//     16-byte load of V (256-byte runs of four rows) feeds four tiles.
+// 128 instructions of 32 cycles per 16 keys and wave, a third of the time HBM needs to bring
+// those keys to a CU. Two waves per SIMD, each with one tile's K and V in registers (the next
+// tile's K is loaded under the softmax and P V, its V under the next Q K), hide each other's
+// loads; holding two tiles per wave instead leaves one wave per SIMD and measured 30 us.
+// B = 8, Hq = 6, S = 4096 as graph replays: 3923 us with one workgroup per sequence, 26.8 now
+// (this kernel 18-20 us, 3.4-3.7 TB/s; the merge 4); B = 16, S = 16384: 99.6 us, 5.4 TB/s.
 constexpr int TAIL_MAXQ = 16;
-constexpr int TAIL_KB = 64;
+constexpr int TAIL_KT = 16;                    // keys per tile
+constexpr int TAIL_NW = 8;                     // waves per workgroup
+constexpr int TAIL_QLD = DH + 4;               // q' rows in LDS, padded off each other's banks
+constexpr float kNegMax = -3.402823466e38f;    // running max before any key: exp(x - m) is 0 or finite
 
-__global__ __launch_bounds__(256) void gqa_tail_kernel(const float* __restrict__ query,
-                                                       const float* __restrict__ gate,
-                                                       const float* __restrict__ q_norm,
-                                                       const float* __restrict__ cos,
-                                                       const float* __restrict__ sin,
-                                                       const float* __restrict__ ck,
-                                                       const float* __restrict__ cv,
-                                                       const float* __restrict__ mask,
-                                                       float* __restrict__ out, int Hq, int S) {
-  const int b = blockIdx.x;
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  __shared__ __attribute__((aligned(16))) float s_q[TAIL_MAXQ][DH];
-  __shared__ float s_p[TAIL_MAXQ][TAIL_KB];
-  __shared__ float s_m[TAIL_MAXQ], s_l[TAIL_MAXQ], s_corr[TAIL_MAXQ];
+struct TailArgs {
+  const float* query;
+  const float* gate;
+  const float* q_norm;
+  const float* cos;
+  const float* sin;
+  const float* ck;
+  const float* cv;
+  const float* mask;
+  float* out;
+  float* po;    // [B][nsplit][Hq][256] unnormalised partial outputs (nsplit > 1)
+  float* pml;   // [B][nsplit][Hq][2] running max and sum
+  int Hq, S, nsplit, per;  // per: 16-key tiles of one split
+};
 
-  // q' rows: wave w prepares rows w, w+4, ...
-  for (int h = w; h < Hq; h += 4) {
-    const float* src = query + ((size_t)b * Hq + h) * DH + 4 * lane;
-    float x[4], ss = 0.f;
-    for (int j = 0; j < 4; ++j) { x[j] = src[j]; ss += x[j] * x[j]; }
-    ss = npn::wave_sum(ss);
-    const float rn = rsqrtf(ss * (1.0f / DH) + kEps);
-    for (int j = 0; j < 4; ++j) x[j] = (1.0f + q_norm[4 * lane + j]) * (x[j] * rn);
-    float y[4];
-    for (int j = 0; j < 4; ++j) y[j] = __shfl_xor(x[j], 8, 64);
-    if (lane < ROPE / 4) {
-      const float sign = lane < ROPE / 8 ? -1.0f : 1.0f;
-      for (int j = 0; j < 4; ++j) x[j] = x[j] * cos[4 * lane + j] + sign * y[j] * sin[4 * lane + j];
-    }
-    for (int j = 0; j < 4; ++j) s_q[h][4 * lane + j] = x[j];
-  }
-  if (tid < Hq) { s_m[tid] = -INFINITY; s_l[tid] = 0.f; }
-  float o[TAIL_MAXQ];
-#pragma unroll
-  for (int h = 0; h < TAIL_MAXQ; ++h) o[h] = 0.f;
-  __syncthreads();
+__global__ __launch_bounds__(64 * TAIL_NW, 2) void gqa_tail_kernel(TailArgs a) {
+  const int b = blockIdx.x / a.nsplit;
+  const int sp = blockIdx.x - b * a.nsplit;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i = lane & 15, g = lane >> 4;
+  const int Hq = a.Hq, S = a.S;
+  __shared__ __attribute__((aligned(16))) float s_o[TAIL_NW][TAIL_MAXQ][DH];
+  __shared__ float s_ml[TAIL_NW][TAIL_MAXQ][2];
+  float (*s_q)[TAIL_QLD] = reinterpret_cast<float (*)[TAIL_QLD]>(&s_o[0][0][0]);
 
-  const float* kb = ck + (size_t)b * S * DH;
-  const float* vb = cv + (size_t)b * S * DH;
-  for (int j0 = 0; j0 < S; j0 += TAIL_KB) {
-    const int nk = S - j0 < TAIL_KB ? S - j0 : TAIL_KB;
-    for (int jj = w; jj < nk; jj += 4) {
-      const float4 kv = reinterpret_cast<const float4*>(kb + (size_t)(j0 + jj) * DH)[lane];
-      const float bias = (1.0f - mask[j0 + jj]) * -1e9f;
-      for (int h = 0; h < Hq; ++h) {
-        const float4 q = reinterpret_cast<const float4*>(s_q[h])[lane];
-        const float s = npn::wave_sum(q.x * kv.x + q.y * kv.y + q.z * kv.z + q.w * kv.w);
-        if (lane == 0) s_p[h][jj] = s * (1.0f / 16.0f) + bias;
-      }
-    }
-    __syncthreads();
-    if (tid < Hq) {
-      float mx = s_m[tid];
-      for (int jj = 0; jj < nk; ++jj) mx = fmaxf(mx, s_p[tid][jj]);
-      const float corr = __expf(s_m[tid] - mx);
-      float l = s_l[tid] * (s_m[tid] == -INFINITY ? 0.f : corr);
-      for (int jj = 0; jj < nk; ++jj) {
-        const float p = __expf(s_p[tid][jj] - mx);
-        s_p[tid][jj] = p;
-        l += p;
-      }
-      s_corr[tid] = s_m[tid] == -INFINITY ? 0.f : corr;
-      s_m[tid] = mx;
-      s_l[tid] = l;
-    }
-    __syncthreads();
+  // The split's tiles of 16 keys, wave w taking every TAIL_NW-th one.
+  const int nt = (S + TAIL_KT - 1) / TAIL_KT;
+  const int t_hi = min(nt, (sp + 1) * a.per);
+  const float* kb = a.ck + (size_t)b * S * DH;
+  const float* vb = a.cv + (size_t)b * S * DH;
+  // Loads of tile t through buffer descriptors over its rows only: rows past S, and every row
+  // when t is past the split, read as 0 without touching memory, so the loads carry no branch
+  // (one would make the compiler wait for a tile's V before its K is used).
+  auto rows_of = [&](const float* base, int t, int row_bytes) {
+    const int rows = t < t_hi ? min(TAIL_KT, S - t * TAIL_KT) : 0;
+    return __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(base + (size_t)t * TAIL_KT * (row_bytes / 4)), (short)0,
+        rows * row_bytes, 0x00020000);
+  };
+  auto load_k = [&](int t, f32x4 (&k)[16]) {
+    const auto r = rows_of(kb, t, DH * 4);
 #pragma unroll
-    for (int h = 0; h < TAIL_MAXQ; ++h)
-      if (h < Hq) o[h] *= s_corr[h];
-    for (int jj = 0; jj < nk; ++jj) {
-      const float v = vb[(size_t)(j0 + jj) * DH + tid];
+    for (int s = 0; s < 16; ++s)
+      k[s] = __builtin_bit_cast(
+          f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, i * DH * 4 + g * 16 + 64 * s, 0, 0));
+  };
+  auto load_v = [&](int t, f32x4 (&v)[4][4], float (&mk)[4]) {
+    const auto rv = rows_of(vb, t, DH * 4), rm = rows_of(a.mask, t, 4);
 #pragma unroll
-      for (int h = 0; h < TAIL_MAXQ; ++h)
-        if (h < Hq) o[h] += s_p[h][jj] * v;
+    for (int r = 0; r < 4; ++r) {
+      mk[r] = __builtin_bit_cast(
+          float, __builtin_amdgcn_raw_buffer_load_b32(rm, 16 * g + 4 * r, 0, 0));
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+        v[r][n] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                rv, (4 * g + r) * DH * 4 + 16 * i + 256 * n, 0, 0));
     }
-    __syncthreads();
-  }
+  };
+
+  // q' rows: wave w prepares rows w and w + 8; rows past Hq are zero. Their loads go out
+  // first, then the first tile's, which land while q' is formed.
+  f32x4 x[TAIL_MAXQ / TAIL_NW];
 #pragma unroll
-  for (int h = 0; h < TAIL_MAXQ; ++h) {
+  for (int u = 0; u < TAIL_MAXQ / TAIL_NW; ++u) {
+    const int h = w + TAIL_NW * u;
+    x[u] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (h < Hq) {
-      const size_t oi = ((size_t)b * Hq + h) * DH + tid;
-      out[oi] = o[h] / s_l[h] * npn::sigmoid(gate[oi]);
+      const float* src = a.query + ((size_t)b * Hq + h) * DH + 4 * lane;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[u][j] = src[j];
     }
   }
+  float nw[4], cs[4] = {1.f, 1.f, 1.f, 1.f}, sn[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) nw[j] = 1.0f + a.q_norm[4 * lane + j];
+  if (lane < ROPE / 4) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      cs[j] = a.cos[4 * lane + j];
+      sn[j] = (lane < ROPE / 8 ? -1.0f : 1.0f) * a.sin[4 * lane + j];
+    }
+  }
+  int t = sp * a.per + w;
+  f32x4 kc[16], v[4][4];
+  float mk[4];
+  load_k(t, kc);
+  asm volatile("" ::: "memory");  // K before V, so that K alone is waited for below
+  load_v(t, v, mk);
+#pragma unroll
+  for (int u = 0; u < TAIL_MAXQ / TAIL_NW; ++u) {
+    const f32x4 xx = x[u] * x[u];
+    const float ss = npn::wave_sum((xx[0] + xx[1]) + (xx[2] + xx[3]));
+    const float rn = rsqrtf(ss * (1.0f / DH) + kEps);
+    f32x4 y;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[u][j] = nw[j] * (x[u][j] * rn);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) y[j] = __shfl_xor(x[u][j], 8, 64);
+    if (lane < ROPE / 4) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[u][j] = x[u][j] * cs[j] + y[j] * sn[j];
+    }
+    *reinterpret_cast<f32x4*>(&s_q[w + TAIL_NW * u][4 * lane]) = x[u];
+  }
+  __syncthreads();
+  f32x4 o[4][4];  // [n][j]: rows 4 g + r = heads, column i = dim 64 n + 4 i + j
+#pragma unroll
+  for (int n = 0; n < 4; ++n)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[n][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = kNegMax, l = 0.f;  // of head i, l this lane's keys only
+  while (t < t_hi) {
+    const int key0 = t * TAIL_KT + 4 * g;  // this lane's keys key0 + r
+    const int tn = t + TAIL_NW;
+    f32x4 acc[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    asm volatile("" ::: "memory");  // q' is read again for each tile: 64 registers less to hold
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      const f32x4 q = *reinterpret_cast<const f32x4*>(&s_q[i][16 * s + 4 * g]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kc[s][j], q[j], acc[j], 0, 0, 0);
+    }
+    load_k(tn, kc);  // kc is free again: the next tile's K under the softmax and P V
+    const f32x4 dot = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    float sc[4], mt = kNegMax;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      sc[r] = key0 + r < S ? dot[r] * (1.0f / 16.0f) + (1.0f - mk[r]) * -1e9f : -INFINITY;
+      mt = fmaxf(mt, sc[r]);
+    }
+    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    if (__any(mt > m)) {
+      const float mn = fmaxf(m, mt);
+      const float corr = __expf(m - mn);
+      m = mn;
+      l *= corr;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float cr = __shfl(corr, 4 * g + r, 64);
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) o[n][j][r] *= cr;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float p = __expf(sc[r] - m);
+      l += p;
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          o[n][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, v[r][n][j], o[n][j], 0, 0, 0);
+    }
+    asm volatile("" ::: "memory");
+    load_v(tn, v, mk);
+    t = tn;
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+
+  // The waves' (m, l, O), added in wave order.
+  __syncthreads();  // every wave is done with q'
+  if (g == 0) {
+    s_ml[w][i][0] = m;
+    s_ml[w][i][1] = l;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (4 * g + r < Hq)
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+        *reinterpret_cast<f32x4*>(&s_o[w][4 * g + r][64 * n + 4 * i]) =
+            f32x4{o[n][0][r], o[n][1][r], o[n][2][r], o[n][3][r]};
+  __syncthreads();
+#pragma unroll 2
+  for (int h = tid >> 8; h < Hq; h += TAIL_NW / 4) {
+    const int d = tid & (DH - 1);
+    float M = kNegMax, L = 0.f, O = 0.f;
+#pragma unroll
+    for (int u = 0; u < TAIL_NW; ++u) M = fmaxf(M, s_ml[u][h][0]);
+#pragma unroll
+    for (int u = 0; u < TAIL_NW; ++u) {
+      const float f = __expf(s_ml[u][h][0] - M);
+      L += f * s_ml[u][h][1];
+      O += f * s_o[u][h][d];
+    }
+    if (a.nsplit == 1) {
+      const size_t oi = ((size_t)b * Hq + h) * DH + d;
+      a.out[oi] = O / L * npn::sigmoid(a.gate[oi]);
+    } else {
+      const size_t row = (size_t)blockIdx.x * Hq + h;
+      a.po[row * DH + d] = O;
+      if (d == 0) {
+        a.pml[2 * row] = M;
+        a.pml[2 * row + 1] = L;
+      }
+    }
+  }
+}
+
+// Log-sum-exp merge of one query row's split partials, in split order within each of four
+// interleaved groups; one 256-thread workgroup per (b, h), wave w taking splits w, w + 4, ...
+// (loads four splits at a time), lane 4 dims.
+__global__ __launch_bounds__(256) void gqa_tail_merge_kernel(TailArgs a) {
+  const int b = blockIdx.x / a.Hq;
+  const int h = blockIdx.x - b * a.Hq;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int n = a.nsplit;
+  __shared__ __attribute__((aligned(16))) f32x4 s_o[4][64];
+  __shared__ float s_ml[4][2];
+  const size_t row0 = (size_t)b * n * a.Hq + h;
+  const float gate = a.gate[((size_t)b * a.Hq + h) * DH + threadIdx.x];
+  float M = kNegMax, L = 0.f;
+  f32x4 O = {0.f, 0.f, 0.f, 0.f};
+  for (int base = w; base < n; base += 16) {
+    float mv[4], lv[4];
+    f32x4 ov[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int sp = base + 4 * j;
+      const size_t row = row0 + (size_t)(sp < n ? sp : base) * a.Hq;
+      mv[j] = a.pml[2 * row];
+      lv[j] = sp < n ? a.pml[2 * row + 1] : 0.f;
+      ov[j] = *reinterpret_cast<const f32x4*>(a.po + row * DH + 4 * lane);
+    }
+    float mn = M;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) mn = fmaxf(mn, mv[j]);
+    const float c = __expf(M - mn);
+    M = mn;
+    L *= c;
+    O *= c;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (base + 4 * j >= n) break;
+      const float f = __expf(mv[j] - M);
+      L += f * lv[j];
+      O += f * ov[j];
+    }
+  }
+  s_o[w][lane] = O;
+  if (lane == 0) {
+    s_ml[w][0] = M;
+    s_ml[w][1] = L;
+  }
+  __syncthreads();
+  float Mx = kNegMax, Ls = 0.f, Os = 0.f;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) Mx = fmaxf(Mx, s_ml[u][0]);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const float f = __expf(s_ml[u][0] - Mx);
+    Ls += f * s_ml[u][1];
+    Os += f * reinterpret_cast<const float*>(s_o[u])[threadIdx.x];
+  }
+  a.out[((size_t)b * a.Hq + h) * DH + threadIdx.x] = Os / Ls * npn::sigmoid(gate);
+}
+
+// 16-key tiles per workgroup: about one workgroup per CU (512 in all measured 35 against 28 us at
+// B = 8, S = 4096: every workgroup pays its own start and merge), each with at least four tiles.
+// The floor of four rather than one tile for each of the eight waves puts small problems on
+// twice the CUs: B = 1, S = 1024 20.3 -> 17.6 us, B = 1, S = 4096 22.1 -> 20.8; two tiles gave
+// 17.4 and 23.
+constexpr int kTailWG = 256, kTailMinTiles = 4;
+int tail_tiles(int B, int S) {
+  const int nt = (S + TAIL_KT - 1) / TAIL_KT;
+  const int n = (kTailWG + B / 2) / B;
+  const int per = n > 1 ? (nt + n - 1) / n : nt;
+  return per > kTailMinTiles ? per : kTailMinTiles;
+}
+int tail_splits(int B, int S) {
+  const int nt = (S + TAIL_KT - 1) / TAIL_KT, per = tail_tiles(B, S);
+  return (nt + per - 1) / per;
+}
+
+bool tail_shape_ok(int B, int Hq, int S) {
+  return B >= 1 && Hq >= 1 && Hq <= TAIL_MAXQ && S >= 1;
 }
 
 struct VerifyPlan {
@@ -973,15 +1192,50 @@ extern "C" int npn_gqa_kv_append(const uint16_t* key, const uint16_t* value, con
   return npn_launch_status();
 }
 
+extern "C" size_t npn_gqa_tail_workspace_size(int B, int q_heads, int S) {
+  if (!tail_shape_ok(B, q_heads, S)) return 0;
+  const size_t n = tail_splits(B, S);
+  // at least 16 bytes, so that 0 means an unsupported shape
+  return n == 1 ? 16 : (size_t)B * n * q_heads * (DH + 2) * sizeof(float);
+}
+
+static int tail_launch(const float* query, const float* gate, const float* q_norm,
+                       const float* cos, const float* sin, const float* cached_k,
+                       const float* cached_v, const float* mask, float* out, int B, int q_heads,
+                       int S, int per, float* ws, void* stream) {
+  NPN_REQUIRE(query && gate && q_norm && cos && sin && cached_k && cached_v && mask && out,
+              NPN_ERR_NULL);
+  NPN_REQUIRE(tail_shape_ok(B, q_heads, S), NPN_ERR_SHAPE);
+  NPN_REQUIRE(NPN_ALIGNED16(cached_k) && NPN_ALIGNED16(cached_v), NPN_ERR_ALIGN);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int nt = (S + TAIL_KT - 1) / TAIL_KT, nsplit = (nt + per - 1) / per;
+  float* pml = nsplit > 1 ? ws + (size_t)B * nsplit * q_heads * DH : nullptr;
+  const TailArgs a{query, gate, q_norm, cos, sin, cached_k, cached_v, mask, out, ws, pml,
+                   q_heads, S, nsplit, per};
+  hipLaunchKernelGGL(gqa_tail_kernel, dim3(B * nsplit), dim3(64 * TAIL_NW), 0, s, a);
+  if (nsplit > 1)
+    hipLaunchKernelGGL(gqa_tail_merge_kernel, dim3(B * q_heads), dim3(256), 0, s, a);
+  return npn_launch_status();
+}
+
 extern "C" int npn_gqa_tail(const float* query, const float* gate, const float* q_norm,
                             const float* cos, const float* sin, const float* cached_k,
                             const float* cached_v, const float* mask, float* out, int B,
                             int q_heads, int S, void* stream) {
-  NPN_REQUIRE(query && gate && q_norm && cos && sin && cached_k && cached_v && mask && out,
-              NPN_ERR_NULL);
-  NPN_REQUIRE(B >= 1 && q_heads >= 1 && q_heads <= TAIL_MAXQ && S >= 1, NPN_ERR_SHAPE);
-  NPN_REQUIRE(NPN_ALIGNED16(cached_k) && NPN_ALIGNED16(cached_v), NPN_ERR_ALIGN);
-  hipLaunchKernelGGL(gqa_tail_kernel, dim3(B), dim3(DH), 0, static_cast<hipStream_t>(stream),
-                     query, gate, q_norm, cos, sin, cached_k, cached_v, mask, out, q_heads, S);
-  return npn_launch_status();
+  return tail_launch(query, gate, q_norm, cos, sin, cached_k, cached_v, mask, out, B, q_heads, S,
+                     S, nullptr, stream);  // S tiles: at least every tile of the sequence
+}
+
+extern "C" int npn_gqa_tail_split(const float* query, const float* gate, const float* q_norm,
+                                  const float* cos, const float* sin, const float* cached_k,
+                                  const float* cached_v, const float* mask, float* out, int B,
+                                  int q_heads, int S, void* workspace, size_t workspace_bytes,
+                                  void* stream) {
+  NPN_REQUIRE(tail_shape_ok(B, q_heads, S), NPN_ERR_SHAPE);
+  NPN_REQUIRE(NPN_ALIGNED16(workspace), NPN_ERR_ALIGN);
+  NPN_REQUIRE(workspace != nullptr &&
+                  workspace_bytes >= npn_gqa_tail_workspace_size(B, q_heads, S),
+              NPN_ERR_WORKSPACE);
+  return tail_launch(query, gate, q_norm, cos, sin, cached_k, cached_v, mask, out, B, q_heads, S,
+                     tail_tiles(B, S), static_cast<float*>(workspace), stream);
 }

@@ -54,9 +54,13 @@ def gqa_tail(
     require(cached_k, "cached_k", torch.float32, shape=(B * S, HEAD_DIM))
     require(cached_v, "cached_v", torch.float32, shape=(B * S, HEAD_DIM))
     require(mask, "mask", torch.float32, numel=S)
+    n_ws = size_query("npn_gqa_tail_workspace_size", B, hq, S)
+    if n_ws == 0:
+        raise RuntimeError(f"unsupported gqa::tail sizes B={B} Hq={hq} S={S}")
+    ws = torch.empty(n_ws, dtype=torch.uint8, device=query.device)
     out = torch.empty_like(query)
-    call("npn_gqa_tail", query, gate, q_norm, cos, sin, cached_k, cached_v, mask, out,
-         B, hq, S, stream_of(query))
+    call("npn_gqa_tail_split", query, gate, q_norm, cos, sin, cached_k, cached_v, mask, out,
+         B, hq, S, ws, n_ws, stream_of(query))
     return out
 
 

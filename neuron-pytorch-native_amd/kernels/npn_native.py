@@ -26,6 +26,8 @@ SIGNATURES = {
     "npn_deltanet_verify": (_I, [_P, _P, _I] + [_P] * 12 + [_I, _I, _I, _I, _P]),
     "npn_deltanet_rollback": (_I, [_P] * 6 + [_I, _I, _I, _I, _P]),
     "npn_gqa_tail": (_I, [_P] * 9 + [_I, _I, _I, _P]),
+    "npn_gqa_tail_workspace_size": (_Z, [_I] * 3),
+    "npn_gqa_tail_split": (_I, [_P] * 9 + [_I, _I, _I, _P, _Z, _P]),
     "npn_gqa_tail_verify_workspace_size": (_Z, [_I] * 5),
     "npn_gqa_tail_verify": (_I, [_P] * 9 + [_I] * 5 + [_P, _Z, _P]),
     "npn_gqa_kv_append": (_I, [_P] * 8 + [_I] * 4 + [_P]),

@@ -38,6 +38,36 @@ def test_tail_reference_shapes(ops):
     assert_rel_close(got.cpu().double().numpy(), ref, name="gqa.tail")
 
 
+@pytest.mark.parametrize("B,HQ,S", [(1, 1, 1), (1, 16, 17), (3, 6, 127), (2, 8, 4100), (5, 3, 64),
+                                    (300, 2, 33)])
+def test_tail_key_splits(ops, B, HQ, S):
+    """gqa::tail over one to 16 heads, partial last key tiles (16 keys), one to 64 splits and one
+    workgroup per sequence, with masked keys anywhere; the workspace-free C entry (always one
+    split) beside it. Each score is an fp32 sum of 256 products of total size about |q'||k| / 16
+    = 16, off by about sqrt(256) 2^-24 16 = 1.5e-5, and so is its weight relative to the others:
+    the bound is six times that. An infinite V entry in the last row, next to the rows that a
+    partial tile clamps to it, stays in its own column."""
+    from npn_native import call, stream_of
+    g = torch.Generator().manual_seed(B + HQ + S)
+    r = lambda *n: torch.randn(*n, generator=g)  # noqa: E731
+    q, gate, ck, cv = r(B * HQ, 256), r(B * HQ, 256), r(B * S, 256), r(B * S, 256)
+    qn, cos, sin = r(1, 256) * 0.1, r(1, 64), r(1, 64)
+    mask = (torch.rand(1, S, generator=g) < 0.7).float()
+    mask[0, S - 1] = 1.0
+    args = (q, gate, qn, cos, sin, ck, cv, mask)
+    ref = og.gqa_tail(*[a.numpy() for a in args])
+    dev = [a.cuda() for a in args]
+    one = torch.empty_like(dev[0])
+    call("npn_gqa_tail", *dev, one, B, HQ, S, stream_of(one))
+    for name, got in (("split", ops.gqa.tail(*dev)), ("one workgroup", one)):
+        assert_rel_close(got.cpu().double().numpy(), ref, tol=1e-4, name=name)
+    dev[6][S - 1, 5] = float("inf")
+    got = ops.gqa.tail(*dev).reshape(B, HQ, 256)[0]
+    assert torch.isposinf(got[:, 5]).all()
+    got[:, 5] = 0
+    assert torch.isfinite(got).all()
+
+
 def _run_verify(ops, d):
     out = ops.gqa.tail_verify(*[d[k].cuda() for k in
                                 ("query", "gate", "q_norm", "cos", "sin", "cache_k", "cache_v",
