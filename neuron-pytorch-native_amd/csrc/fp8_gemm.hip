@@ -1339,11 +1339,58 @@ void plan_wide128(int M, GemmPlan& p) {
   }
 }
 
+// Plan for more than 256 rows, where the grid usually takes several rounds of 256 workgroups:
+// the (kernel, tile width, split-K factor) with the least modelled time
+//   rounds x (64-k chunks x (a + b x units per workgroup) + e) + partial traffic
+// in us. The constants are a least-squares fit to 4,600 timings on MI355X (seven projection
+// shapes, 64 < M <= 3584, weights rotated through 400 MB, 5 % rms); its choice was within 1 %
+// of the best of all configurations on average. The rule before (each row pass planned as if
+// it were alone, 128-row tiles only when they fitted one round) left the last round nearly
+// empty or tiled 16 columns at a time: M = 4096 17408 x 5120 1600 -> 583 us, M = 700 5120 x
+// 16512 191 -> 112, M = 2048 5120 x 8704 282 -> 171, M = 2048 5120 x 34816 689 -> 601. Split-K
+// partials stay under 64 MB (they are written and read back through the memory-side cache).
+void plan_rows(int M, int K, int N, GemmPlan& p) {
+  const int units = N / 16;
+  double best = 1e30;
+  auto offer = [&](bool rows128, int nh, bool odd, int per, int s) {
+    const int groups = (units + per - 1) / per;
+    const int rtiles = rows128 ? (M + 127) / 128 : (M + 255) / 256;
+    const long wgs = (long)groups * rtiles * s;
+    const int chunks = (K / KC + s - 1) / s;
+    const double step = rows128 ? 0.226 + 0.0422 * per : 0.333 + 0.0741 * per;
+    double t = (double)((wgs + WIDE_WG - 1) / WIDE_WG) * (chunks * step + 1.75);
+    if (s > 1) t += 2.0 * s * M * N * 4 / 4.9e6 + 2.0;
+    if (t >= best) return;
+    best = t;
+    p.wide = true;
+    p.rows128 = rows128;
+    p.odd = odd;
+    p.ntm = nh;
+    p.h128 = rows128 ? per / 2 : 0;
+    p.units = units;
+    p.groups = groups;
+    p.split_k = s;
+  };
+  for (int s = 1; s <= 8 && K / KC >= 2 * s; s *= 2) {
+    if (s > 1 && (double)s * M * N * 4 > 64e6) break;
+    for (const Wide128Cfg& c : kWide128) offer(true, c.nh, c.odd, 4 * c.nh - (c.odd ? 2 : 0), s);
+    for (int v : kWideNH) offer(false, v, false, 2 * v, s);
+  }
+  p.passes = (M + 255) / 256;
+  p.ualign = 1;
+  p.ws = p.split_k > 1 ? (size_t)p.split_k * M * N * sizeof(float) : 0;
+}
+
 GemmPlan plan(int M, int K, int N, bool no_split = false, int ua = 1) {
   GemmPlan p{};
   if (plan_wide(M, K, N, p, no_split, ua)) {
     // the argmax and chunk-statistics epilogues exist only in the 256-row kernel
-    if (!no_split && ua == 1) plan_wide128(M, p);
+    if (!no_split && ua == 1) {
+      plan_wide128(M, p);
+      // up to three 128-row tiles a one-round plan of the 128-row kernel is within 10 % of the
+      // model's choice (5120 x 14336 71 against 63 us, 17408 x 5120 75 against 77)
+      if (M > 256 && !(p.rows128 && M <= 384)) plan_rows(M, K, N, p);
+    }
     return p;
   }
   p = GemmPlan{};

@@ -171,6 +171,40 @@ def test_rows128_plans(ops, M, K, N, S, U):
                      out_unit=BF16_ULP, name=f"fp8 rows128 M={M} K={K} N={N}")
 
 
+@pytest.mark.parametrize("M,K,N,plan", [
+    (385, 128, 34816, (3, 1, 18)), (4096, 128, 64, (3, 1, 4)), (4095, 128, 5120, (3, 1, 20)),
+    (1025, 192, 8704, (3, 1, 20)), (700, 128, 16512, (2, 1, 7)), (2300, 128, 34816, (2, 1, 7)),
+    (513, 17408, 640, (3, 8, 8)), (770, 17408, 1344, (3, 4, 10)), (1200, 17408, 5120, (2, 2, 7))])
+def test_many_row_plans(ops, M, K, N, plan):
+    """More than 256 rows: both wide kernels in one and several rounds of workgroups, with and
+    without split-K, partial row tiles and column groups. Unsplit plans equal the 256-row
+    kernel's one-pass-at-a-time plan (npn_fp8_matmul_rowmax) bit for bit, with the SwiGLU
+    epilogue too; every plan against the oracle on sampled columns and rows."""
+    from npn_native import call, query, stream_of
+    kind, split, tile, _ = _plan(M, K, N)
+    assert (kind, split, tile) == plan
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w, scale = fp8_weights(N, K, seed=N + 3)
+    xd, wd, sd = x.cuda(), w.cuda(), scale.reshape(N, 1).cuda()
+    got = ops.fp8.matmul(xd, wd, sd)
+    if split == 1:
+        ref = torch.empty_like(got)
+        gmax = torch.empty((M, query("npn_fp8_matmul_argmax_groups", M, K, N)), device="cuda")
+        call("npn_fp8_matmul_rowmax", xd, wd, sd, ref, gmax, M, K, N, stream_of(xd))
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+        if N % 128 == 0:
+            act = ops.fp8.matmul_swiglu(xd, wd, sd)
+            assert torch.equal(act.view(torch.int16), ops.glue.silu_mul(ref).view(torch.int16))
+    rng = np.random.default_rng(N)
+    cols = np.unique(np.concatenate([[0, N - 1], rng.choice(N, min(N, 192), replace=False)]))
+    rows = np.unique(np.concatenate([[0, M - 1], rng.choice(M, 256, replace=False)]))
+    ref = of.fp8_matmul(bits(x)[rows], w.numpy()[:, cols], scale.numpy()[cols])
+    assert_rel_close(got.float().cpu().double().numpy()[np.ix_(rows, cols)], round_to_bf16(ref),
+                     out_unit=BF16_ULP, name=f"fp8 M={M} K={K} N={N}")
+
+
 @pytest.mark.parametrize("M,N", [(8, 5120), (64, 17408), (256, 34816)])
 def test_verify_shapes_sampled(ops, M, N):
     rng = np.random.default_rng(M)
