@@ -183,7 +183,7 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
     tile -= ka.tiles1;
   }
   constexpr int NTH = NWV * 64;
-  constexpr int CH = NWV / RB;               // column slices
+  constexpr int CH = NWV;                    // column slices, one per wave
   constexpr int CB = 16 / CH;                // columns (bytes) per lane
   static_assert(CB >= 4 && CB <= 16, "4 to 16 columns per lane");
   constexpr int WST = 32 * NT;               // W stage bytes
@@ -199,14 +199,15 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int i = lane & 15, G = lane >> 4;
-  const int rb = w / CH, ch = w - rb * CH;
+  const int ch = w;
   const int nks = a.K / KSTEP;
-  const int mrow = m_pass + 16 * rb + i;              // A operand row of this lane
-  const bool row_ok = mrow < a.M;
+  bool row_ok[RB];                                    // A operand rows of this lane
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) row_ok[rb] = m_pass + 16 * rb + i < a.M;
   const int lcol = ch * 16 * CB + CB * i;             // the lane's first column in the tile
 
   // k steps ks_lo .. ks_lo + ntile - 1 of the tile at column n0, summed into acc.
-  auto run = [&](int n0, int ks_lo, int ntile, f32x4 (&acc)[CB]) {
+  auto run = [&](int n0, int ks_lo, int ntile, f32x4 (&acc)[RB][CB]) {
     // DMA of k step ks into stage st: W rows (WQ x 16 bytes per thread), then x rows.
     auto issue = [&](int ks, int st) {
       uint8_t* ws = smem + st * STAGE;
@@ -243,9 +244,13 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
       if (tn < ntile) issue(ks_lo + tn, tn % NS);
       const uint8_t* ws = smem + (t % NS) * STAGE;
       const uint8_t* xs = ws + WST;
-      const u32x4 xv = *reinterpret_cast<const u32x4*>(xs + (16 * rb + i) * 64 + 16 * G);
-      const u32x4 zero = {0u, 0u, 0u, 0u};
-      const bf16x8 aop = __builtin_bit_cast(bf16x8, row_ok ? xv : zero);
+      bf16x8 aop[RB];
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        const u32x4 xv = *reinterpret_cast<const u32x4*>(xs + (16 * rb + i) * 64 + 16 * G);
+        const u32x4 zero = {0u, 0u, 0u, 0u};
+        aop[rb] = __builtin_bit_cast(bf16x8, row_ok[rb] ? xv : zero);
+      }
       uint32_t d[8][CB / 4];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -271,8 +276,10 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
         transpose_dequant(dq, bop);
 #pragma unroll
         for (int ct = 0; ct < 4; ++ct)
-          acc[4 * q + ct] =
-              __builtin_amdgcn_mfma_f32_16x16x32_bf16(aop, bop[ct], acc[4 * q + ct], 0, 0, 0);
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb)
+            acc[rb][4 * q + ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                aop[rb], bop[ct], acc[rb][4 * q + ct], 0, 0, 0);
       }
     }
     // (every DMA has landed: the last tile waited with vmcnt(0))
@@ -280,21 +287,23 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
 
   // fp32 sums (unscaled) of this lane's rows and columns of the tile at n0 into partial
   // slot `slot` ([split_k][M][N]); zero sums when `zero`.
-  auto store_partial = [&](int slot, int n0, const f32x4 (&acc)[CB], bool zero) {
+  auto store_partial = [&](int slot, int n0, const f32x4 (&acc)[RB][CB], bool zero) {
     const int nc = n0 + lcol;
     if (nc >= a.N) return;
     float* part = a.partial + (size_t)slot * a.M * a.N;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m_pass + 16 * rb + 4 * G + r;
-      if (m >= a.M) continue;
-      float4* dst = reinterpret_cast<float4*>(part + (size_t)m * a.N + nc);
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-      for (int c = 0; c < CB / 4; ++c)
-        dst[c] = zero ? make_float4(0.f, 0.f, 0.f, 0.f)
-                      : make_float4(acc[4 * c][r], acc[4 * c + 1][r], acc[4 * c + 2][r],
-                                    acc[4 * c + 3][r]);
-    }
+      for (int r = 0; r < 4; ++r) {
+        const int m = m_pass + 16 * rb + 4 * G + r;
+        if (m >= a.M) continue;
+        float4* dst = reinterpret_cast<float4*>(part + (size_t)m * a.N + nc);
+#pragma unroll
+        for (int c = 0; c < CB / 4; ++c)
+          dst[c] = zero ? make_float4(0.f, 0.f, 0.f, 0.f)
+                        : make_float4(acc[rb][4 * c][r], acc[rb][4 * c + 1][r],
+                                      acc[rb][4 * c + 2][r], acc[rb][4 * c + 3][r]);
+      }
   };
 
   if (a.sk_wg > 0) {
@@ -313,9 +322,11 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
       const int hi = (int)(u1 - tb < nks ? u1 - tb : nks);
       const int wfirst = (int)(((tb + 1) * W - 1) / U);
       const int wlast = (int)(((tb + nks) * W - 1) / U);
-      f32x4 acc[CB];
+      f32x4 acc[RB][CB];
 #pragma unroll
-      for (int c = 0; c < CB; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int c = 0; c < CB; ++c) acc[rb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
       __syncthreads();  // every wave is done with the ring's previous segment
       run((int)t * NT, lo, hi - lo, acc);
       store_partial((int)wg - wfirst, (int)t * NT, acc, false);
@@ -330,9 +341,11 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
   const int sk = blockIdx.y;
   const int ks_lo = (int)(((long)nks * sk) / a.split_k);
   const int ks_hi = (int)(((long)nks * (sk + 1)) / a.split_k);
-  f32x4 acc[CB];
+  f32x4 acc[RB][CB];
 #pragma unroll
-  for (int c = 0; c < CB; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int c = 0; c < CB; ++c) acc[rb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   run(n0, ks_lo, ks_hi - ks_lo, acc);
 
 
@@ -347,13 +360,14 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
 #pragma unroll
     for (int c = 0; c < CB; ++c) sc[c] = col_ok ? a.scale[nc + c] : 0.0f;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
+    for (int rr = 0; rr < 4 * RB; ++rr) {
+      const int rb = rr >> 2, r = rr & 3;
       float bv = -__builtin_inff();
       int bi = 0x7FFFFFFF;
       if (col_ok) {
 #pragma unroll
         for (int c = 0; c < CB; ++c) {
-          const float v = bf16_round(acc[c][r] * sc[c]);
+          const float v = bf16_round(acc[rb][c][r] * sc[c]);
           if (arg_beats(v, nc + c, bv, bi)) {
             bv = v;
             bi = nc + c;
@@ -371,14 +385,15 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
 #pragma unroll
     for (int c = 0; c < CB; ++c) sc[c] = col_ok ? a.scale[nc + c] : 0.0f;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
+    for (int rr = 0; rr < 4 * RB; ++rr) {
+      const int rb = rr >> 2, r = rr & 3;
       const int m = m_pass + 16 * rb + 4 * G + r;
       uint32_t pk[CB / 2];
       float mx = -__builtin_inff();  // max of the row's bf16 outputs (fmaxf ignores NaN)
 #pragma unroll
       for (int c = 0; c < CB / 2; ++c) {
-        const uint32_t lo = npn::f32_to_bf16(acc[2 * c][r] * sc[2 * c]);
-        const uint32_t hi = npn::f32_to_bf16(acc[2 * c + 1][r] * sc[2 * c + 1]);
+        const uint32_t lo = npn::f32_to_bf16(acc[rb][2 * c][r] * sc[2 * c]);
+        const uint32_t hi = npn::f32_to_bf16(acc[rb][2 * c + 1][r] * sc[2 * c + 1]);
         pk[c] = lo | (hi << 16);
         mx = fmaxf(mx, fmaxf(npn::bf16_to_f32(lo), npn::bf16_to_f32(hi)));
       }
@@ -1442,7 +1457,7 @@ GemmPlan plan(int M, int K, int N, bool no_split = false, int ua = 1) {
 
 // Column slices per narrow tile (the kernel's CH = waves / row blocks): its row-maximum and
 // argmax groups are (tile, slice) pairs.
-int narrow_slices(int mt) { return mt == 1 ? 4 : (mt == 2 ? 4 : 2); }
+int narrow_slices(int) { return 4; }
 
 bool shape_ok(int M, int K, int N) {
   return M >= 1 && M <= 4096 && K >= 64 && K % 64 == 0 && N >= 64 && N % 64 == 0 &&
@@ -1502,8 +1517,8 @@ int launch_gemm(const GemmPlan& p, const uint16_t* x, const int8_t* w, const flo
     const dim3 grid = p.sk_wg > 0 ? dim3(p.sk_wg, 1, 1) : dim3((N + NT - 1) / NT, p.split_k, p.passes);
     switch (p.mt) {
       case 1: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<1, 4, 4>), grid, dim3(256), 0, s, ga); break;
-      case 2: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<2, 4, 8>), grid, dim3(512), 0, s, ga); break;
-      default: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<4, 4, 8>), grid, dim3(512), 0, s, ga); break;
+      case 2: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<2, 4, 4>), grid, dim3(256), 0, s, ga); break;
+      default: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<4, 4, 4>), grid, dim3(256), 0, s, ga); break;
     }
   }
   if (reduce && p.split_k > 1) {
@@ -1533,8 +1548,8 @@ bool launch_gemm_pair_partials(const uint16_t* x, const int8_t* w1, float* p1, i
   const dim3 grid(t1 + t2, a.split_k, 1);
   switch (a.mt) {
     case 1: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<1, 4, 4>), grid, dim3(256), 0, s, ga); break;
-    case 2: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<2, 4, 8>), grid, dim3(512), 0, s, ga); break;
-    default: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<4, 4, 8>), grid, dim3(512), 0, s, ga); break;
+    case 2: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<2, 4, 4>), grid, dim3(256), 0, s, ga); break;
+    default: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<4, 4, 4>), grid, dim3(256), 0, s, ga); break;
   }
   return true;
 }
