@@ -42,6 +42,7 @@ struct DnArgs {
   uint16_t* out;
   int B, T, Hk, Hv;
   int nsplit;  // workgroups per head, each storing 128 / nsplit of the head's columns
+  uint16_t* conv_out;  // T == 1: the shifted conv window [B][QKV][3] (nullptr: not written)
 };
 
 // Depthwise causal conv (4 taps, oldest first) + bias + SiLU of channel c over T tokens.
@@ -138,6 +139,16 @@ __global__ __launch_bounds__(128 * P) void dn_verify_kernel(DnArgs a) {
       conv_channel<TMAX>(csb, xb, a.conv_weight, a.conv_bias, chan, QKV, T, y);
 #pragma unroll
       for (int t = 0; t < TMAX; ++t) dst[t][i] = y[t];
+      // The single-token window shift [cs1, cs2, x] of the channels this workgroup owns: its
+      // head's v, and the group's q and k when it is the group's first head.
+      if (TMAX == 1 && a.conv_out != nullptr && split == 0 &&
+          (which == 2 || h == kh * (a.Hv / a.Hk))) {
+        const uint16_t* cs = csb + (size_t)chan * 3;
+        uint16_t* co = a.conv_out + ((size_t)b * QKV + chan) * 3;
+        co[0] = cs[1];
+        co[1] = cs[2];
+        co[2] = xb[chan];
+      }
     }
   }
   if (tid < T) {
@@ -352,15 +363,13 @@ int verify_impl(const DnArgs& a, hipStream_t s) {
   return npn_launch_status();
 }
 
-}  // namespace
-
-extern "C" int npn_deltanet_verify(const float* state, const int32_t* state_index, int state_T,
-                                   const uint16_t* mixed_qkv, const uint16_t* conv_state,
-                                   const float* conv_weight, const float* conv_bias,
-                                   const float* a_out, const float* b_out, const uint16_t* z,
-                                   const float* A_log, const float* dt_bias,
-                                   const float* norm_weight, float* ckpt, uint16_t* out, int B,
-                                   int T, int k_heads, int v_heads, void* stream) {
+// npn_deltanet_verify, and with conv_out (T == 1) the window shift in the same launch.
+int verify_checked(const float* state, const int32_t* state_index, int state_T,
+                   const uint16_t* mixed_qkv, const uint16_t* conv_state,
+                   const float* conv_weight, const float* conv_bias, const float* a_out,
+                   const float* b_out, const uint16_t* z, const float* A_log,
+                   const float* dt_bias, const float* norm_weight, float* ckpt, uint16_t* out,
+                   uint16_t* conv_out, int B, int T, int k_heads, int v_heads, void* stream) {
   NPN_REQUIRE(state && mixed_qkv && conv_state && conv_weight && conv_bias && a_out && b_out &&
                   z && A_log && dt_bias && norm_weight && ckpt && out,
               NPN_ERR_NULL);
@@ -371,8 +380,22 @@ extern "C" int npn_deltanet_verify(const float* state, const int32_t* state_inde
   NPN_REQUIRE(NPN_ALIGNED16(state) && NPN_ALIGNED16(ckpt), NPN_ERR_ALIGN);
   DnArgs a{state, state_index, state_T, mixed_qkv, conv_state, conv_weight, conv_bias,
            a_out,  b_out,       z,       A_log,     dt_bias,    norm_weight, ckpt,
-           out,    B,           T,       k_heads,   v_heads};
+           out,    B,           T,       k_heads,   v_heads,   1,           conv_out};
   return verify_impl(a, static_cast<hipStream_t>(stream));
+}
+
+}  // namespace
+
+extern "C" int npn_deltanet_verify(const float* state, const int32_t* state_index, int state_T,
+                                   const uint16_t* mixed_qkv, const uint16_t* conv_state,
+                                   const float* conv_weight, const float* conv_bias,
+                                   const float* a_out, const float* b_out, const uint16_t* z,
+                                   const float* A_log, const float* dt_bias,
+                                   const float* norm_weight, float* ckpt, uint16_t* out, int B,
+                                   int T, int k_heads, int v_heads, void* stream) {
+  return verify_checked(state, state_index, state_T, mixed_qkv, conv_state, conv_weight,
+                        conv_bias, a_out, b_out, z, A_log, dt_bias, norm_weight, ckpt, out,
+                        nullptr, B, T, k_heads, v_heads, stream);
 }
 
 extern "C" int npn_deltanet_full_batched(const float* state, const uint16_t* mixed_qkv,
@@ -384,15 +407,24 @@ extern "C" int npn_deltanet_full_batched(const float* state, const uint16_t* mix
                                          uint16_t* new_conv_state, uint16_t* out, int B,
                                          int k_heads, int v_heads, void* stream) {
   NPN_REQUIRE(new_conv_state != nullptr, NPN_ERR_NULL);
-  int st = npn_deltanet_verify(state, nullptr, 0, mixed_qkv, conv_state, conv_weight, conv_bias,
-                               a_out, b_out, z, A_log, dt_bias, norm_weight, new_state, out, B,
-                               1, k_heads, v_heads, stream);
-  if (st != NPN_OK) return st;
-  const int QKV = (2 * k_heads + v_heads) * D;
-  const size_t n = (size_t)B * QKV;
+  const size_t n = B > 0 && k_heads > 0 && v_heads > 0
+                       ? (size_t)B * (2 * (size_t)k_heads + v_heads) * D
+                       : 0;
+  // The window shift goes with the verify launch: as a graph node of its own it cost 1.6 us
+  // (calls in one graph, 4/12 heads: B = 1 7.1 -> 5.5 us, B = 8 7.6 -> 5.9, B = 64 18.7 -> 17.7;
+  // 16/48 heads: B = 1 7.4 -> 5.7, B = 8 12.7 -> 11.2). A caller's window that overlaps its input keeps the second launch: a group's
+  // heads all read the q and k windows that its first head would overwrite.
+  const uintptr_t c0 = reinterpret_cast<uintptr_t>(conv_state);
+  const uintptr_t n0 = reinterpret_cast<uintptr_t>(new_conv_state);
+  const bool overlap = n0 < c0 + 6 * n && c0 < n0 + 6 * n;
+  const int st = verify_checked(state, nullptr, 0, mixed_qkv, conv_state, conv_weight, conv_bias,
+                                a_out, b_out, z, A_log, dt_bias, norm_weight, new_state, out,
+                                overlap ? nullptr : new_conv_state, B, 1, k_heads, v_heads,
+                                stream);
+  if (st != NPN_OK || !overlap) return st;
   hipLaunchKernelGGL(dn_conv_window_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), conv_state, mixed_qkv, nullptr,
-                     new_conv_state, B, 1, QKV);
+                     new_conv_state, B, 1, (2 * k_heads + v_heads) * D);
   return npn_launch_status();
 }
 

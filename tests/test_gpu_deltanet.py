@@ -18,6 +18,10 @@ from _util import (assert_rel_close, bits, deltanet_flat_device, deltanet_inputs
 pytestmark = pytest.mark.gpu
 
 
+def bits_t(t):
+    return t.view(torch.int16)
+
+
 def _verify_gpu(ops, d):
     f = deltanet_flat_device(d)
     ckpt, out = ops.deltanet.verify_batched(
@@ -80,6 +84,33 @@ def test_full_batched_reference_shapes(ops, B):
             f["norm_weight"])
         torch.cuda.synchronize()
         assert torch.equal(s1, ns) and torch.equal(c1, ncs) and torch.equal(o1, o)
+
+
+@pytest.mark.parametrize("B,Hk,Hv,overlapping", [
+    (1, 16, 48, False),   # four workgroups per head store a share each
+    (2, 3, 3, False),     # every head is its group's first
+    (33, 16, 48, False),  # two row parts
+    (2, 4, 12, True),     # window shifted in place: a launch of its own
+])
+def test_token_step_shifts_conv_window(ops, B, Hk, Hv, overlapping):
+    """The token step's new window is [conv_state[:, 1:] | x] for every channel, bit for bit,
+    and its state and output are the one-token verify's."""
+    from npn_native import call, stream_of
+    f = deltanet_flat_device(deltanet_inputs(B, 1, Hk, Hv, seed=B + Hv))
+    QKV = (2 * Hk + Hv) * 128
+    want = torch.cat([f["conv_state"].reshape(B, QKV, 3)[:, :, 1:],
+                      f["mixed_qkv"].reshape(B, QKV, 1)], -1).reshape(-1, 3)
+    ckpt, vout = ops.deltanet.verify_batched(*f.values())
+    if overlapping:
+        state, out = torch.empty_like(ckpt), torch.empty_like(vout)
+        conv = f["conv_state"]
+        call("npn_deltanet_full_batched", *f.values(), state, conv, out, B, Hk, Hv,
+             stream_of(state))
+    else:
+        state, conv, out = ops.deltanet.full_batched(*f.values())
+    torch.cuda.synchronize()
+    assert torch.equal(bits_t(conv), bits_t(want))
+    assert torch.equal(state, ckpt) and torch.equal(bits_t(out), bits_t(vout))
 
 
 def test_rollback_copy_and_index(ops):
