@@ -13,6 +13,8 @@
 // with v_cvt_scalef32_pk_bf16_fp8 (exact: every e4m3fn value is a bf16 value). Above 64 rows
 // (the wide kernel, MFMA-bound) the B operands are read back transposed (ds_read_b64_tr_b8)
 // and converted the same way; details with each kernel below.
+#include <type_traits>
+
 #include "accept_contract.h"
 #include "npn_internal.h"
 
@@ -128,7 +130,7 @@ struct GemmArgs {
   // stream-K): column tiles [0, tiles1) are w's, the rest w2's [K, N2] with partials2
   const uint8_t* w2;
   float* partial2;
-  int N2, tiles1;
+  int N2, tiles1, split2;
 };
 
 __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
@@ -146,16 +148,21 @@ __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
 // workgroups). So a workgroup owns a 256-column tile, and each k step's W tile (32 rows x
 // 256 columns, 256-byte row runs) and x rows (16 RB rows x 32 k) move HBM -> LDS by direct
 // loads (global_load_lds_dwordx4), NS stages deep: every W byte is fetched once per
-// workgroup, whatever its number of row blocks, and NS - 1 tiles are in flight. The NWV waves
-// split the tile by rows and columns with no k split: RB row blocks of 16 rows x CH = NWV / RB
-// column slices of 256 / CH columns; lane (i, G) reads CB = 16 / CH bytes (columns) from each
-// of its 8 k rows 8 G + j out of LDS, and each 4-column quarter is transposed and dequantised
-// in registers into the B operands of 4 MFMAs (column ct of quarter q feeds MFMA 4 q + ct).
+// workgroup, whatever its number of row blocks, and NS - 1 tiles are in flight. Four waves
+// (column slices of 64) own all RB blocks of 16 rows: lane (i, G) reads 4 adjacent bytes
+// (columns) from each of its 8 k rows 8 G + j out of LDS, which are transposed and dequantised
+// in registers into the B operands of 4 MFMAs per row block.
+// KG k groups of four waves: with 2, a stage holds 64 k, each group takes 32 of them, and the
+// second group's sums are added to the first's through LDS at the end. One workgroup per CU
+// then has two waves per SIMD to cover the chain of waits, LDS reads, conversions and MFMAs
+// that bounds it (the DMA alone runs 17408 x 5120 in 17 us on 240 workgroups).
 // Each wave issues the same DMA instructions for every tile, so a vmcnt of (tiles issued
 // after tile t) x (this wave's DMAs per tile) names "tile t landed"; an s_barrier then
 // publishes it. For wide N, K is also split across workgroups (split_k); partials then go
-// through an fp32 workspace and a fixed-order reduction kernel.
+// through an fp32 workspace and a fixed-order reduction kernel. The stream-K form is a kernel
+// of its own: its 64-bit share arithmetic cost the others 0.3 to 0.5 us before their first DMA.
 constexpr int NT = 256;     // columns per narrow tile
+constexpr int NS = 4;       // stages of the narrow ring
 
 // s_waitcnt vmcnt(pend * DPT) for a wave-uniform pend in [0, C] (the count is an immediate).
 template <int C, int DPT>
@@ -171,48 +178,55 @@ __device__ __forceinline__ void wait_tiles(int pend) {
   }
 }
 
-template <int RB, int NS, int NWV>
-__global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs ka) {
+template <int RB, int KG, bool STREAM>
+__global__ __launch_bounds__(KG * 256, KG) void fp8_gemm_narrow_kernel(GemmArgs ka) {
+  static_assert(KG == 1 || !STREAM, "stream-K runs one k group");
   // A two-matrix launch runs the second matrix's tiles with its pointers and width.
   GemmArgs a = ka;
   int tile = blockIdx.x;
-  if (ka.tiles1 > 0 && tile >= ka.tiles1) {
-    a.w = ka.w2;
-    a.N = ka.N2;
-    a.partial = ka.partial2;
-    tile -= ka.tiles1;
+  if (!STREAM && ka.tiles1 > 0) {
+    if (tile >= ka.tiles1) {
+      a.w = ka.w2;
+      a.N = ka.N2;
+      a.partial = ka.partial2;
+      a.split_k = ka.split2;
+      tile -= ka.tiles1;
+    }
+    if ((int)blockIdx.y >= a.split_k) return;
   }
-  constexpr int NTH = NWV * 64;
-  constexpr int CH = NWV;                    // column slices, one per wave
+  constexpr int NTH = KG * 256;
+  constexpr int NK = KG * KSTEP;             // k per stage (one k unit)
+  constexpr int CH = 4;                      // column slices, one per wave of a k group
   constexpr int CB = 16 / CH;                // columns (bytes) per lane
-  static_assert(CB >= 4 && CB <= 16, "4 to 16 columns per lane");
-  constexpr int WST = 32 * NT;               // W stage bytes
-  constexpr int XST = 16 * RB * 64;          // x stage bytes (rows x 32 k bf16)
+  constexpr int WST = NK * NT;               // W stage bytes
+  constexpr int XST = 16 * RB * NK * 2;      // x stage bytes, [16 RB rows][32 k] bf16 per group
   constexpr int STAGE = WST + XST;
   constexpr int WQ = WST / 16 / NTH;         // W DMA instructions (16 bytes) per thread
   constexpr int XW = XST / 16 / 64;          // waves that move x, one 16-byte DMA per lane
-  static_assert(WQ * 16 * NTH == WST && XW * 64 * 16 == XST && XW <= NWV,
+  static_assert(WQ * 16 * NTH == WST && XW * 64 * 16 == XST && XW <= NTH / 64,
                 "whole DMA instructions per stage");
+  static_assert(KG == 1 || NS * STAGE >= RB * CB * 256 * 16, "the ring holds a group's sums");
   __shared__ __attribute__((aligned(16))) uint8_t smem[NS * STAGE];
 
   const int m_pass = blockIdx.z * 16 * RB;
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int i = lane & 15, G = lane >> 4;
-  const int ch = w;
-  const int nks = a.K / KSTEP;
+  const int ch = w & 3, kg = KG == 1 ? 0 : w >> 2;
+  const int nku = a.K / NK;
   bool row_ok[RB];                                    // A operand rows of this lane
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) row_ok[rb] = m_pass + 16 * rb + i < a.M;
   const int lcol = ch * 16 * CB + CB * i;             // the lane's first column in the tile
 
-  // k steps ks_lo .. ks_lo + ntile - 1 of the tile at column n0, summed into acc.
-  auto run = [&](int n0, int ks_lo, int ntile, f32x4 (&acc)[RB][CB]) {
-    // DMA of k step ks into stage st: W rows (WQ x 16 bytes per thread), then x rows.
-    auto issue = [&](int ks, int st) {
+  // k units lo .. lo + ntile - 1 of the tile at column n0, summed into acc; the whole sums are
+  // in the first k group's waves.
+  auto run = [&](int n0, int lo, int ntile, f32x4 (&acc)[RB][CB]) {
+    // DMA of k unit ku into stage st: W rows (WQ x 16 bytes per thread), then x rows.
+    auto issue = [&](int ku, int st) {
       uint8_t* ws = smem + st * STAGE;
       uint8_t* xs = ws + WST;
-      const int k0 = ks * KSTEP;
+      const int k0 = ku * NK;
 #pragma unroll
       for (int q = 0; q < WQ; ++q) {
         const int s = q * NTH + tid;                  // 16-byte slot of the W stage
@@ -222,15 +236,15 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
         npn::lds_dma16(a.w + (size_t)(k0 + row) * a.N + col, ws + q * (NTH * 16) + (tid & ~63) * 16);
       }
       if (w < XW) {                                   // 16-byte slots, 4 per 64-byte row
-        const int s = w * 64 + lane;
-        int m = m_pass + (s >> 2);
+        const int xh = w / RB;                        // the k group whose k the slot holds
+        int m = m_pass + (((w - xh * RB) * 64 + lane) >> 2);
         m = m < a.M ? m : a.M - 1;
-        npn::lds_dma16(a.x + (size_t)m * a.K + k0 + 8 * (s & 3), xs + w * 1024);
+        npn::lds_dma16(a.x + (size_t)m * a.K + k0 + KSTEP * xh + 8 * (lane & 3), xs + w * 1024);
       }
     };
 #pragma unroll
     for (int p = 0; p < NS - 1; ++p)
-      if (p < ntile) issue(ks_lo + p, p);
+      if (p < ntile) issue(lo + p, p);
     for (int t = 0; t < ntile; ++t) {
       // Tiles t + 1 .. min(t + NS - 2, ntile - 1) were issued after tile t: wait until at
       // most their DMAs are outstanding (this wave's count per tile is WQ, plus one x DMA
@@ -241,9 +255,9 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       const int tn = t + NS - 1;                      // into the stage tile t - 1 used
-      if (tn < ntile) issue(ks_lo + tn, tn % NS);
-      const uint8_t* ws = smem + (t % NS) * STAGE;
-      const uint8_t* xs = ws + WST;
+      if (tn < ntile) issue(lo + tn, tn % NS);
+      const uint8_t* ws = smem + (t % NS) * STAGE + kg * (KSTEP * NT);
+      const uint8_t* xs = smem + (t % NS) * STAGE + WST + kg * (RB * 1024);
       bf16x8 aop[RB];
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
@@ -251,38 +265,37 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
         const u32x4 zero = {0u, 0u, 0u, 0u};
         aop[rb] = __builtin_bit_cast(bf16x8, row_ok[rb] ? xv : zero);
       }
-      uint32_t d[8][CB / 4];
+      uint32_t d[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const uint8_t* src = ws + (8 * G + j) * NT + lcol;
-        if constexpr (CB == 16) {
-          const u32x4 v = *reinterpret_cast<const u32x4*>(src);
+      for (int j = 0; j < 8; ++j)
+        d[j] = *reinterpret_cast<const uint32_t*>(ws + (8 * G + j) * NT + lcol);
+      bf16x8 bop[4];
+      transpose_dequant(d, bop);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) d[j][q] = v[q];
-        } else if constexpr (CB == 8) {
-          const uint2 v = *reinterpret_cast<const uint2*>(src);
-          d[j][0] = v.x;
-          d[j][1] = v.y;
-        } else {
-          d[j][0] = *reinterpret_cast<const uint32_t*>(src);
-        }
-      }
+      for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
-      for (int q = 0; q < CB / 4; ++q) {
-        uint32_t dq[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) dq[j] = d[j][q];
-        bf16x8 bop[4];
-        transpose_dequant(dq, bop);
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-          for (int rb = 0; rb < RB; ++rb)
-            acc[rb][4 * q + ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                aop[rb], bop[ct], acc[rb][4 * q + ct], 0, 0, 0);
-      }
+        for (int rb = 0; rb < RB; ++rb)
+          acc[rb][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aop[rb], bop[ct], acc[rb][ct],
+                                                                0, 0, 0);
     }
     // (every DMA has landed: the last tile waited with vmcnt(0))
+    if constexpr (KG == 2) {  // the second group's sums pass through the ring to the first's
+      f32x4* xch = reinterpret_cast<f32x4*>(smem) + (tid & 255);
+      __syncthreads();
+      if (kg == 1) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+          for (int c = 0; c < CB; ++c) xch[(rb * CB + c) * 256] = acc[rb][c];
+      }
+      __syncthreads();
+      if (kg == 0) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+          for (int c = 0; c < CB; ++c) acc[rb][c] += xch[(rb * CB + c) * 256];
+      }
+    }
   };
 
   // fp32 sums (unscaled) of this lane's rows and columns of the tile at n0 into partial
@@ -290,71 +303,84 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
   auto store_partial = [&](int slot, int n0, const f32x4 (&acc)[RB][CB], bool zero) {
     const int nc = n0 + lcol;
     if (nc >= a.N) return;
-    float* part = a.partial + (size_t)slot * a.M * a.N;
+    int m = m_pass + 4 * G;
+    float* dst = a.partial + ((size_t)slot * a.M + m) * a.N + nc;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (m + r < a.M)
+          *reinterpret_cast<float4*>(dst + (size_t)r * a.N) =
+              zero ? make_float4(0.f, 0.f, 0.f, 0.f)
+                   : make_float4(acc[rb][0][r], acc[rb][1][r], acc[rb][2][r], acc[rb][3][r]);
+      }
+      m += 16;
+      dst += (size_t)16 * a.N;
+    }
+  };
+
+  // The workgroup's run [u0, u1) of k units, the tiles' units laid end to end: its (tile, k
+  // split) share, inside one tile, or with stream-K over W workgroups an equal run of all U
+  // units, units [wg U / W, (wg + 1) U / W). There a tile's units are covered by workgroups
+  // wfirst .. wlast (closed form: the workgroup that holds unit x is ((x + 1) W - 1) / U);
+  // workgroup wg writes its sums of tile t to slot wg - wfirst, and wlast zeroes the slots past
+  // the tile's last, so every tile's split_k slots add to its full sum in slot order.
+  const bool partials = STREAM || a.to_partial || (a.split_k > 1 && a.amax == nullptr);
+  const int wg = blockIdx.x;
+  int lo, hi;
+  long W = 0, U = 0, u1 = 0;
+  if constexpr (STREAM) {
+    W = a.sk_wg;
+    U = (long)((a.N + NT - 1) / NT) * nku;
+    const long u0 = wg * U / W;
+    u1 = (wg + 1) * U / W;
+    tile = (int)(u0 / nku);
+    lo = (int)(u0 - (long)tile * nku);
+    hi = (int)min(u1 - (long)tile * nku, (long)nku);
+  } else {  // the first nku % split_k splits take a unit more
+    const int sk = blockIdx.y, per = nku / a.split_k, more = nku - per * a.split_k;
+    lo = per * sk + min(sk, more);
+    hi = lo + per + (sk < more ? 1 : 0);
+  }
+  f32x4 acc[RB][CB];
+  for (;;) {
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = m_pass + 16 * rb + 4 * G + r;
-        if (m >= a.M) continue;
-        float4* dst = reinterpret_cast<float4*>(part + (size_t)m * a.N + nc);
-#pragma unroll
-        for (int c = 0; c < CB / 4; ++c)
-          dst[c] = zero ? make_float4(0.f, 0.f, 0.f, 0.f)
-                        : make_float4(acc[rb][4 * c][r], acc[rb][4 * c + 1][r],
-                                      acc[rb][4 * c + 2][r], acc[rb][4 * c + 3][r]);
-      }
-  };
-
-  if (a.sk_wg > 0) {
-    // Stream-K: the tiles' k steps laid end to end (U units), workgroup wg taking units
-    // [wg U / W, (wg + 1) U / W). A tile's units are covered by workgroups wfirst .. wlast
-    // (closed form: the workgroup that holds unit x is ((x + 1) W - 1) / U); workgroup wg
-    // writes its sums of tile t to slot wg - wfirst, and wlast zeroes the slots past the
-    // tile's last, so every tile's split_k slots add to its full sum in slot order.
-    const long U = (long)((a.N + NT - 1) / NT) * nks;
-    const long W = a.sk_wg;
-    const long wg = blockIdx.x;
-    const long u0 = wg * U / W, u1 = (wg + 1) * U / W;
-    for (long t = u0 / nks; t * nks < u1; ++t) {
-      const long tb = t * nks;
-      const int lo = (int)(u0 > tb ? u0 - tb : 0);
-      const int hi = (int)(u1 - tb < nks ? u1 - tb : nks);
+      for (int c = 0; c < CB; ++c) acc[rb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    run(tile * NT, lo, hi - lo, acc);
+    if (!partials) break;
+    if (kg != 0) return;
+    if constexpr (!STREAM) {
+      store_partial(blockIdx.y, tile * NT, acc, false);
+      return;
+    } else {
+      const long tb = (long)tile * nku;
       const int wfirst = (int)(((tb + 1) * W - 1) / U);
-      const int wlast = (int)(((tb + nks) * W - 1) / U);
-      f32x4 acc[RB][CB];
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int c = 0; c < CB; ++c) acc[rb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-      __syncthreads();  // every wave is done with the ring's previous segment
-      run((int)t * NT, lo, hi - lo, acc);
-      store_partial((int)wg - wfirst, (int)t * NT, acc, false);
+      const int wlast = (int)(((tb + nku) * W - 1) / U);
+      store_partial(wg - wfirst, tile * NT, acc, false);
       if (wg == wlast)
         for (int sl = wlast - wfirst + 1; sl < a.split_k; ++sl)
-          store_partial(sl, (int)t * NT, acc, true);
+          store_partial(sl, tile * NT, acc, true);
+      if (tb + nku >= u1) return;
+      ++tile;
+      lo = 0;
+      hi = (int)min(u1 - tb - nku, (long)nku);
+      __syncthreads();  // every wave is done with the ring's previous segment
     }
-    return;
   }
+  if (kg != 0) return;
 
-  const int n0 = tile * NT;
-  const int sk = blockIdx.y;
-  const int ks_lo = (int)(((long)nks * sk) / a.split_k);
-  const int ks_hi = (int)(((long)nks * (sk + 1)) / a.split_k);
-  f32x4 acc[RB][CB];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-    for (int c = 0; c < CB; ++c) acc[rb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  run(n0, ks_lo, ks_hi - ks_lo, acc);
-
-
-  // Lane (i, G) holds rows m_pass + 16 rb + 4 G + r and columns nc + c in acc[c][r]; its
-  // group for the row maxima is the (tile, column slice) pair.
-  const int nc = n0 + lcol;
+  // Lane (i, G) holds rows m_pass + 16 rb + 4 G + r and columns nc + c in acc[rb][c][r]. The
+  // row maxima's groups are GM adjacent slices of the tile (narrow_slices).
+  constexpr int GM = RB == 4 ? 2 : 1;
+  const int nc = tile * NT + lcol;
   const bool col_ok = nc < a.N;
-  const int groups = gridDim.x * CH;
-  const int grp = blockIdx.x * CH + ch;
+  const int groups = gridDim.x * (CH / GM);
+  const int grp = blockIdx.x * (CH / GM) + ch / GM;
+  // [16 RB rows][4 slices] when GM == 2, once every wave is done with the ring
+  ArgPart* pair = reinterpret_cast<ArgPart*>(smem);
+  if constexpr (GM == 2) __syncthreads();
   if (a.amax != nullptr) {
     float sc[CB];
 #pragma unroll
@@ -375,73 +401,83 @@ __global__ __launch_bounds__(NWV * 64, 1) void fp8_gemm_narrow_kernel(GemmArgs k
         }
       }
       arg_merge16(bv, bi);
-      const int m = m_pass + 16 * rb + 4 * G + r;
-      if (i == 0 && m < a.M) a.amax[(size_t)m * groups + grp] = ArgPart{bv, bi};
+      const int row = 16 * rb + 4 * G + r, m = m_pass + row;
+      if (i == 0) {
+        if constexpr (GM == 2) pair[row * CH + ch] = ArgPart{bv, bi};
+        else if (m < a.M) a.amax[(size_t)m * groups + grp] = ArgPart{bv, bi};
+      }
+    }
+    if constexpr (GM == 2) {                          // 64 rows x 2 groups
+      __syncthreads();
+      const int row = tid >> 1, m = m_pass + row;
+      if (tid < 128 && m < a.M) {
+        const ArgPart p = pair[row * CH + 2 * (tid & 1)], q = pair[row * CH + 2 * (tid & 1) + 1];
+        a.amax[(size_t)m * groups + blockIdx.x * 2 + (tid & 1)] = arg_beats(q.v, q.i, p.v, p.i) ? q : p;
+      }
     }
     return;
   }
-  if (a.split_k == 1 && !a.to_partial) {
-    float sc[CB];
+  float sc[CB];
 #pragma unroll
-    for (int c = 0; c < CB; ++c) sc[c] = col_ok ? a.scale[nc + c] : 0.0f;
+  for (int c = 0; c < CB; ++c) sc[c] = col_ok ? a.scale[nc + c] : 0.0f;
 #pragma unroll
-    for (int rr = 0; rr < 4 * RB; ++rr) {
-      const int rb = rr >> 2, r = rr & 3;
-      const int m = m_pass + 16 * rb + 4 * G + r;
-      uint32_t pk[CB / 2];
-      float mx = -__builtin_inff();  // max of the row's bf16 outputs (fmaxf ignores NaN)
+  for (int rr = 0; rr < 4 * RB; ++rr) {
+    const int rb = rr >> 2, r = rr & 3;
+    const int m = m_pass + 16 * rb + 4 * G + r;
+    uint32_t pk[CB / 2];
+    float mx = -__builtin_inff();  // max of the row's bf16 outputs (fmaxf ignores NaN)
 #pragma unroll
-      for (int c = 0; c < CB / 2; ++c) {
-        const uint32_t lo = npn::f32_to_bf16(acc[rb][2 * c][r] * sc[2 * c]);
-        const uint32_t hi = npn::f32_to_bf16(acc[rb][2 * c + 1][r] * sc[2 * c + 1]);
-        pk[c] = lo | (hi << 16);
-        mx = fmaxf(mx, fmaxf(npn::bf16_to_f32(lo), npn::bf16_to_f32(hi)));
-      }
-      if (col_ok && m < a.M) {
-        uint16_t* dst = a.out + (size_t)m * a.N + nc;
-        if constexpr (CB == 16) {
-          reinterpret_cast<uint4*>(dst)[0] = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-          reinterpret_cast<uint4*>(dst)[1] = make_uint4(pk[4], pk[5], pk[6], pk[7]);
-        } else if constexpr (CB == 8) {
-          *reinterpret_cast<uint4*>(dst) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-        } else {
-          *reinterpret_cast<uint2*>(dst) = make_uint2(pk[0], pk[1]);
-        }
-      }
-      if (a.gmax != nullptr) {  // the 16 lanes of a group share the row; lanes past N add -inf
-        if (!col_ok) mx = -__builtin_inff();
+    for (int c = 0; c < CB / 2; ++c) {
+      const uint32_t lo = npn::f32_to_bf16(acc[rb][2 * c][r] * sc[2 * c]);
+      const uint32_t hi = npn::f32_to_bf16(acc[rb][2 * c + 1][r] * sc[2 * c + 1]);
+      pk[c] = lo | (hi << 16);
+      mx = fmaxf(mx, fmaxf(npn::bf16_to_f32(lo), npn::bf16_to_f32(hi)));
+    }
+    if (col_ok && m < a.M) {
+      uint16_t* dst = a.out + (size_t)m * a.N + nc;
+      *reinterpret_cast<uint2*>(dst) = make_uint2(pk[0], pk[1]);
+    }
+    if (a.gmax != nullptr) {  // the 16 lanes of a group share the row; lanes past N add -inf
+      if (!col_ok) mx = -__builtin_inff();
 #pragma unroll
-        for (int off = 8; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-        if (i == 0 && m < a.M) a.gmax[(size_t)m * groups + grp] = mx;
-      }
-      if (a.cmax != nullptr) {
-        // Contract chunk statistics: a 64-column chunk is held by LPC adjacent lanes of the
-        // 16-lane group (N % 64 == 0, so a chunk is wholly inside or wholly past N).
-        constexpr int LPC = 64 / CB;  // 16, 8 or 4: a DPP row, half-row or quad
-        constexpr int STEPS = LPC == 16 ? 4 : (LPC == 8 ? 3 : 2);
-        float xs[CB];
-#pragma unroll
-        for (int c = 0; c < CB / 2; ++c) {
-          xs[2 * c] = npn::scaled(npn::bf16lo(pk[c]), a.inv_temp);
-          xs[2 * c + 1] = npn::scaled(npn::bf16hi(pk[c]), a.inv_temp);
-        }
-        float cmx = -__builtin_inff();
-#pragma unroll
-        for (int c = 0; c < CB; ++c) cmx = fmaxf(cmx, xs[c]);
-        cmx = npn::row_max_dpp<STEPS>(cmx);
-        uint64_t csm = 0;
-#pragma unroll
-        for (int c = 0; c < CB; ++c) csm += npn::expfix_rel(xs[c], cmx);
-        csm = npn::row_sum_dpp<STEPS>(csm);
-        if (i % LPC == 0 && col_ok && m < a.M) {
-          const size_t o = (size_t)m * (a.N / 64) + (nc >> 6);
-          a.cmax[o] = cmx;
-          a.csum[o] = csm;
-        }
+      for (int off = 8; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+      if (i == 0) {
+        if constexpr (GM == 2) pair[(16 * rb + 4 * G + r) * CH + ch].v = mx;
+        else if (m < a.M) a.gmax[(size_t)m * groups + grp] = mx;
       }
     }
-  } else {
-    store_partial(sk, n0, acc, false);
+    if (a.cmax != nullptr) {
+      // Contract chunk statistics: a 64-column chunk is held by LPC adjacent lanes of the
+      // 16-lane group (N % 64 == 0, so a chunk is wholly inside or wholly past N).
+      constexpr int LPC = 64 / CB;  // 16, 8 or 4: a DPP row, half-row or quad
+      constexpr int STEPS = LPC == 16 ? 4 : (LPC == 8 ? 3 : 2);
+      float xs[CB];
+#pragma unroll
+      for (int c = 0; c < CB / 2; ++c) {
+        xs[2 * c] = npn::scaled(npn::bf16lo(pk[c]), a.inv_temp);
+        xs[2 * c + 1] = npn::scaled(npn::bf16hi(pk[c]), a.inv_temp);
+      }
+      float cmx = -__builtin_inff();
+#pragma unroll
+      for (int c = 0; c < CB; ++c) cmx = fmaxf(cmx, xs[c]);
+      cmx = npn::row_max_dpp<STEPS>(cmx);
+      uint64_t csm = 0;
+#pragma unroll
+      for (int c = 0; c < CB; ++c) csm += npn::expfix_rel(xs[c], cmx);
+      csm = npn::row_sum_dpp<STEPS>(csm);
+      if (i % LPC == 0 && col_ok && m < a.M) {
+        const size_t o = (size_t)m * (a.N / 64) + (nc >> 6);
+        a.cmax[o] = cmx;
+        a.csum[o] = csm;
+      }
+    }
+  }
+  if (GM == 2 && a.gmax != nullptr) {
+    __syncthreads();
+    const int row = tid >> 1, m = m_pass + row;
+    if (tid < 128 && m < a.M)
+      a.gmax[(size_t)m * groups + blockIdx.x * 2 + (tid & 1)] =
+          fmaxf(pair[row * CH + 2 * (tid & 1)].v, pair[row * CH + 2 * (tid & 1) + 1].v);
   }
 }
 
@@ -1430,6 +1466,14 @@ GemmPlan plan(int M, int K, int N, bool no_split = false, int ua = 1) {
   while (!no_split && p.split_k < max_split && tiles * p.split_k * 2 <= max_wg &&
          nks >= 16 * p.split_k)
     p.split_k *= 2;
+  // From 21 tiles the powers of two put between one and three workgroups on a CU (272 for 34
+  // tiles x 8: 16 CUs do twice the work of the rest); the grid of one per CU does better
+  // although it streams with fewer waves: K = 5120, GEMM and reduction, N = 8704 split 16 -> 7
+  // at 8 rows 17.4 -> 15.7 us, split 8 -> 7 at 40 rows 27.5 -> 18.7 (with two k groups);
+  // N = 10240 split 16 -> 6 at 16 rows 20.9 -> 16.8; N = 13824 24.1 -> 21.2. Up to 20 tiles 16
+  // splits of a few rows measured the same, and from 55 tiles stream-K takes over.
+  if (!no_split && tiles * p.split_k > WIDE_WG && tiles > 20 && tiles <= 54)
+    p.split_k = WIDE_WG / tiles;
   // Stream-K where the tiles x split grid cannot fill the CUs evenly (136 tiles x 4 = 544
   // workgroups leave 32 CUs with three while the rest run two): up to 512 workgroups (two per
   // CU) share the tiles' k steps equally, at least 8 each, with at most 8 partial slots per
@@ -1455,13 +1499,40 @@ GemmPlan plan(int M, int K, int N, bool no_split = false, int ua = 1) {
   return p;
 }
 
-// Column slices per narrow tile (the kernel's CH = waves / row blocks): its row-maximum and
-// argmax groups are (tile, slice) pairs.
-int narrow_slices(int) { return 4; }
+// Row-maximum and argmax groups per 256-column narrow tile, by its row blocks.
+int narrow_slices(int mt) { return mt == 4 ? 2 : 4; }
 
 bool shape_ok(int M, int K, int N) {
   return M >= 1 && M <= 4096 && K >= 64 && K % 64 == 0 && N >= 64 && N % 64 == 0 &&
          (long)K * N < (1L << 40);
+}
+
+// Whether a narrow plan of N columns runs the two-k-group form: more than 16 rows, and at most
+// one workgroup per CU. Two groups feed a lone workgroup's SIMDs with two waves each (17408 x
+// 5120 in 160 workgroups, GEMM and reduction: 32 rows 36.6 -> 26.7 us, 64 rows 50.9 -> 32.9);
+// where CUs hold two workgroups already they only cost (64 rows 5120 x 34816 in 512: 64 -> 95,
+// 16 rows 5120 x 4608 in 288: 14.2 -> 15.3). Up to 16 rows the gain is small (256 workgroups
+// 5 %), and one form for all of them keeps the two matrices of a pair launch together.
+bool two_groups(const GemmPlan& p, int N) {
+  return p.mt > 1 && p.sk_wg == 0 &&
+         (long)((N + NT - 1) / NT) * p.split_k * p.passes <= WIDE_WG;
+}
+
+void launch_narrow(const GemmArgs& ga, int mt, bool two, dim3 grid, hipStream_t s) {
+  auto go = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, ga);
+  };
+  auto pick = [&](auto rb) {
+    constexpr int RB = decltype(rb)::value;
+    if (ga.sk_wg > 0) go(fp8_gemm_narrow_kernel<RB, 1, true>, 256);
+    else if constexpr (RB > 1) {
+      if (two) go(fp8_gemm_narrow_kernel<RB, 2, false>, 512);
+      else go(fp8_gemm_narrow_kernel<RB, 1, false>, 256);
+    } else go(fp8_gemm_narrow_kernel<RB, 1, false>, 256);
+  };
+  if (mt == 1) pick(std::integral_constant<int, 1>{});
+  else if (mt == 2) pick(std::integral_constant<int, 2>{});
+  else pick(std::integral_constant<int, 4>{});
 }
 
 // Launches the plan's GEMM kernel; with split-K (or to_partial) it writes fp32 partials
@@ -1515,11 +1586,7 @@ int launch_gemm(const GemmPlan& p, const uint16_t* x, const int8_t* w, const flo
     GemmArgs ga{x, reinterpret_cast<const uint8_t*>(w), scale, out, partial, M, K, N, p.split_k,
                 to_partial, amax, gmax, p.sk_wg, cmax, csum, inv_temp};
     const dim3 grid = p.sk_wg > 0 ? dim3(p.sk_wg, 1, 1) : dim3((N + NT - 1) / NT, p.split_k, p.passes);
-    switch (p.mt) {
-      case 1: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<1, 4, 4>), grid, dim3(256), 0, s, ga); break;
-      case 2: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<2, 4, 4>), grid, dim3(256), 0, s, ga); break;
-      default: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<4, 4, 4>), grid, dim3(256), 0, s, ga); break;
-    }
+    launch_narrow(ga, p.mt, two_groups(p, N), grid, s);
   }
   if (reduce && p.split_k > 1) {
     const size_t total = (size_t)M * N;
@@ -1529,28 +1596,20 @@ int launch_gemm(const GemmPlan& p, const uint16_t* x, const int8_t* w, const flo
   return npn_launch_status();
 }
 
-// The split-K partials of two GEMMs of the same x ([M, K], M <= 64) in one narrow launch,
-// W1 [K, N1] into p1 [S][M][N1] and W2 [K, N2] into p2 [S][M][N2]: the same tiles, k ranges
-// and sums as two launches of their plans, which must be narrow tiles x split grids with one
-// pass and the same row blocks and split-K factor S. Returns false (nothing launched) when
-// they are not.
+// The split-K partials of two GEMMs of the same x ([M, K], M <= 16) in one narrow launch, W1
+// [K, N1] into p1 [S1][M][N1] and W2 [K, N2] into p2 [S2][M][N2]: the same tiles, k ranges and
+// sums as two launches of their plans, which must be narrow tiles x split grids of one pass.
+// Returns false (nothing launched) when they are not.
 bool launch_gemm_pair_partials(const uint16_t* x, const int8_t* w1, float* p1, int N1,
                                const int8_t* w2, float* p2, int N2, int M, int K,
                                hipStream_t s) {
   const GemmPlan a = plan(M, K, N1), b = plan(M, K, N2);
-  if (a.wide || b.wide || a.sk_wg > 0 || b.sk_wg > 0 || a.passes != 1 || b.passes != 1 ||
-      a.mt != b.mt || a.split_k != b.split_k)
-    return false;
+  if (M > 16 || a.sk_wg > 0 || b.sk_wg > 0) return false;
   const int t1 = (N1 + NT - 1) / NT, t2 = (N2 + NT - 1) / NT;
   GemmArgs ga{x, reinterpret_cast<const uint8_t*>(w1), nullptr, nullptr, p1, M, K, N1,
               a.split_k, 1, nullptr, nullptr, 0, nullptr, nullptr, 1.0f,
-              reinterpret_cast<const uint8_t*>(w2), p2, N2, t1};
-  const dim3 grid(t1 + t2, a.split_k, 1);
-  switch (a.mt) {
-    case 1: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<1, 4, 4>), grid, dim3(256), 0, s, ga); break;
-    case 2: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<2, 4, 4>), grid, dim3(256), 0, s, ga); break;
-    default: hipLaunchKernelGGL((fp8_gemm_narrow_kernel<4, 4, 4>), grid, dim3(256), 0, s, ga); break;
-  }
+              reinterpret_cast<const uint8_t*>(w2), p2, N2, t1, b.split_k};
+  launch_narrow(ga, a.mt, false, dim3(t1 + t2, std::max(a.split_k, b.split_k), 1), s);
   return true;
 }
 

@@ -55,6 +55,23 @@ def test_stream_k(ops, M, K, N):
     _check(ops, M, K, N, seed=K + N)
 
 
+@pytest.mark.parametrize("M,K,N,S", [
+    (17, 64, 320, 1),      # one k unit, partial last tile, two k groups
+    (33, 832, 5120, 2),    # 13 k units over two splits
+    (64, 1728, 1088, 4),   # 27 k units over four splits
+    (32, 5120, 4096, 8),   # 128 workgroups
+    (16, 5120, 5632, 11),  # 22 tiles: one workgroup per CU, one k group
+    (40, 5120, 8704, 7),   # 34 tiles: the same with two k groups
+    (24, 2560, 13824, 4),  # 54 tiles
+])
+def test_one_workgroup_per_cu(ops, M, K, N, S):
+    """Narrow grids of at most one workgroup per CU: the split-K factor that fills the CUs, and
+    above 16 rows the form with two k groups per workgroup, every column checked."""
+    import npn_native
+    assert npn_native.query("npn_fp8_matmul_split_k", M, K, N) == S
+    _check(ops, M, K, N, seed=K + N)
+
+
 @pytest.mark.parametrize("M,K,N", [(8, 17408, 5120), (16, 6144, 4608)])
 def test_split_16(ops, M, K, N):
     """At most 16 rows with few 256-column tiles: split-K 16, every column checked."""
