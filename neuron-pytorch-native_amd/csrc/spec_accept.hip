@@ -370,12 +370,6 @@ __device__ __forceinline__ u256 map256(u256 v, F f) {
               ((uint64_t)w[5] << 32) | w[4], ((uint64_t)w[7] << 32) | w[6]};
 }
 
-__device__ __forceinline__ u256 shfl_u256(u256 v, int src) {
-  return map256(v, [&](uint32_t x) { return (uint32_t)__shfl(x, src, 64); });
-}
-__device__ __forceinline__ u256 shfl_up_u256(u256 v, int d) {
-  return map256(v, [&](uint32_t x) { return (uint32_t)__shfl_up(x, d, 64); });
-}
 __device__ __forceinline__ u256 shfl_xor_u256(u256 v, int m) {
   return map256(v, [&](uint32_t x) { return (uint32_t)__shfl_xor(x, m, 64); });
 }
@@ -394,15 +388,27 @@ __device__ __forceinline__ u256 wave_sum_u256(u256 v) {
   return add256(v, shfl_xor_u256(v, 32));
 }
 
-// Inclusive prefix sum over the 64 lanes of a wave.
+// Inclusive prefix sum over the 64 lanes of a wave, by DPP moves: shifts by 1, 2, 4 and 8 inside
+// each 16-lane row, then the last lane of row 0 (2) into row 1 (3), and of row 1 into rows 2 and
+// 3. Lanes without a source add 0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ u256 scan_step_u256(u256 v) {
+  return add256(v, map256(v, [](uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xF, true);
+  }));
+}
 __device__ __forceinline__ u256 wave_incl_scan_u256(u256 v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const u256 o = shfl_up_u256(v, d);
-    if (lane >= d) v = add256(v, o);
-  }
-  return v;
+  v = scan_step_u256<0x111, 0xF>(v);  // row_shr:1
+  v = scan_step_u256<0x112, 0xF>(v);
+  v = scan_step_u256<0x114, 0xF>(v);
+  v = scan_step_u256<0x118, 0xF>(v);
+  v = scan_step_u256<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
+  return scan_step_u256<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
+}
+
+// Lane src's value (src the same in every lane).
+__device__ __forceinline__ u256 read_lane_u256(u256 v, int src) {
+  return map256(v, [&](uint32_t x) { return (uint32_t)__builtin_amdgcn_readlane((int)x, src); });
 }
 
 __device__ __forceinline__ u128 wave_sum_u128(u128 v) {
@@ -677,13 +683,14 @@ struct DecideSmem {
   Decision d;
 };
 
-// Row totals and the decision of sequence b, by a whole THREADS-wide workgroup: each 16-lane
+// Row totals and the decision of sequence b, by a whole NTH-wide workgroup: each 16-lane
 // row of lanes takes one of the sequence's 2K+1 rows at a time, lane l its blocks l, l + 16, ...:
 // M = max_b M_b, Z = sum_b G_b S_b (G_b = expfix(M_b - M)), and the weight of the row's draft
 // token W = (E F) G_b from the statistics pass's E F. Then lane i < K of wave 0 runs the
 // accept test of position i (all at once; the first failing lane is the rejection). With
 // `write` it also stores every row's Z and M, the decision record, accepted[b] and out_ids but
 // the sampled token. Ends with a barrier, after which sm.d holds the decision.
+template <int NTH>
 __device__ void decide_sequence(const RejArgs& a, int b, bool write, DecideSmem& sm) {
   const int K = a.K, T = K + 1, nt = a.B * T;
   const int t = threadIdx.x, lane = t & 63, gl = t & 15;
@@ -693,7 +700,7 @@ __device__ void decide_sequence(const RejArgs& a, int b, bool write, DecideSmem&
     id = a.draft_ids[(size_t)b * K + t];
     u = a.u_accept[(size_t)b * K + t];
   }
-  for (int j = t >> 4; j < T + K; j += THREADS / 16) {
+  for (int j = t >> 4; j < T + K; j += NTH / 16) {
     const int row = j < T ? b * T + j : nt + b * K + (j - T);
     const int tok = row_token(a, row);
     const uint64_t ef = a.tw[row];  // issued with the other loads; 0 without a token
@@ -710,7 +717,10 @@ __device__ void decide_sequence(const RejArgs& a, int b, bool write, DecideSmem&
     const float M = npn::row_max_dpp<4>(mx);
     u128 z = 0;
 #pragma unroll
-    for (int k = 0; k < kDecideBlocksPerLane; ++k) z += bs[k] * expfix_rel(bm[k], M);
+    for (int k = 0; k < kDecideBlocksPerLane; ++k) {
+      if (16 * k >= a.nb) break;  // (no lane has a block)
+      z += bs[k] * expfix_rel(bm[k], M);
+    }
     z = row_sum_u128(z);
     // M_b of the token's block: lane tb & 15 of the row holds it in bm[tb >> 4]
     const int tb = tok >= 0 ? tok / npn::kContractBlock : 0;
@@ -937,38 +947,65 @@ __device__ __forceinline__ float chunk_max(const float (&v)[N]) {
 // Residual (or bonus) mass per contract chunk and per 2048-entry sub-chunk of the sampling rows.
 // Every workgroup first works out its sequence's decision (block statistics only; workgroup
 // x == 0 writes it out), then block x covers the contract block x of the sampling rows, each
-// wave one sub-chunk, each lane a run of 32 entries, the lanes 2c, 2c + 1 of a wave forming
-// chunk c of its sub-chunk (whose maxima they reduce between them). The chunk masses go to
-// cm64 and the wave's sum to cmass; no workgroup reads another's results (the pick kernel,
-// launched after this one, does).
-constexpr int MRUN = MCHK / 64;  // entries per lane of the mass kernel
-static_assert(2 * MRUN == CC, "two lanes per contract chunk");
-
-template <bool kUnitTemp, typename TT>
-__global__ __launch_bounds__(THREADS) void rej_mass_kernel(RejArgs a) {
+// lane a run of MRUN entries, CC / MRUN adjacent lanes forming a chunk (whose maxima they reduce
+// between them). The chunk masses go to cm64 and the sub-chunks' sums to cmass; no workgroup
+// reads another's results (the pick kernel, launched after this one, does).
+// Grids of many workgroups take runs of 32 entries (4 waves a block, a wave one sub-chunk): the
+// wide products are per run, so longer runs do fewer of them. Up to MASS_WG workgroups the
+// chip has room and the time is one wave's chain, so runs of 8 spread a block over 16 waves
+// (B = 8, V = 151936, 152 workgroups: 13.2 -> 10.5 to 11.8 us; the whole call with the pick's
+// scans by DPP, 9.0 -> 6.5 to 7.3 us, 39.6 -> 34.1). Runs of 32 stay for more: B = 32, 608
+// workgroups of them, 19.4 us.
+constexpr int MASS_WG = 256;
+template <bool kUnitTemp, typename TT, int MRUN>
+__global__ __launch_bounds__(npn::kContractBlock / MRUN) void rej_mass_kernel(RejArgs a) {
+  constexpr int NTH = npn::kContractBlock / MRUN;
+  constexpr int LANES = CC / MRUN;               // lanes per chunk: 2 or 8
+  constexpr int WPS = MCHK / (64 * MRUN);        // waves per sub-chunk: 1 or 4
   __shared__ DecideSmem sm;
+  __shared__ u256 s_w[NTH / 64];
   const int b = (int)blockIdx.y;
-  decide_sequence(a, b, blockIdx.x == 0, sm);
-  const int lane = threadIdx.x & 63;
-  const int sub = (int)blockIdx.x * (THREADS / 64) + (int)(threadIdx.x >> 6);
-  if (sub >= a.nchm) return;  // the whole wave
+  decide_sequence<NTH>(a, b, blockIdx.x == 0, sm);
+  const int lane = threadIdx.x & 63, w = (int)(threadIdx.x >> 6);
   const Decision d = sm.d;
   const int K = a.K, T = K + 1, nt = a.B * T;
   const int rp = b * T + d.acc, rq = nt + b * K + d.acc;
   const TT* p = target_row<TT>(a, rp);
   const float* q = d.acc < K ? a.draft + (size_t)(b * K + d.acc) * a.V : nullptr;
-  const float Mbp = a.bmax[(size_t)rp * a.nb + blockIdx.x];
-  const float Mbq = q != nullptr ? a.bmax[(size_t)rq * a.nb + blockIdx.x] : 0.f;
-  const int v0 = sub * MCHK + lane * MRUN;
-  const RunVals<MRUN> rv = load_run<MRUN, kUnitTemp>(a, p, q, v0);
-  const float mpc = chunk_max<2>(rv.p), mqc = chunk_max<2>(rv.q);
-  u256 m = kZero256;
-  if (v0 < a.V) m = run_mass<MRUN>(sample_row<TT>(d, p, q, mpc, mqc, Mbp, Mbq), rv);
-  const u256 mc = add256(m, dpp_u256<npn::kDppStep[0]>(m));  // lanes 2c and 2c + 1
-  const int c = v0 / CC;
-  if ((lane & 1) == 0 && c < a.nc) a.cm64[(size_t)b * a.nc + c] = mc;
-  m = wave_sum_u256(m);
-  if (lane == 0) a.cmass[(size_t)b * a.nchm + sub] = m;
+  const int v0 = (int)blockIdx.x * npn::kContractBlock + (int)threadIdx.x * MRUN;
+  if (v0 - lane * MRUN < a.V) {                  // the whole wave
+    const float Mbp = a.bmax[(size_t)rp * a.nb + blockIdx.x];
+    const float Mbq = q != nullptr ? a.bmax[(size_t)rq * a.nb + blockIdx.x] : 0.f;
+    const RunVals<MRUN> rv = load_run<MRUN, kUnitTemp>(a, p, q, v0);
+    const float mpc = chunk_max<LANES>(rv.p), mqc = chunk_max<LANES>(rv.q);
+    u256 m = kZero256;
+    if (v0 < a.V) m = run_mass<MRUN>(sample_row<TT>(d, p, q, mpc, mqc, Mbp, Mbq), rv);
+    u256 mc = add256(m, dpp_u256<npn::kDppStep[0]>(m));
+    if constexpr (LANES == 8) {
+      mc = add256(mc, dpp_u256<npn::kDppStep[1]>(mc));
+      mc = add256(mc, dpp_u256<npn::kDppStep[2]>(mc));
+    }
+    const int c = v0 / CC;
+    if (lane % LANES == 0 && c < a.nc) a.cm64[(size_t)b * a.nc + c] = mc;
+    m = wave_sum_u256(m);
+    if (lane == 0) {
+      if constexpr (WPS == 1) a.cmass[(size_t)b * a.nchm + v0 / MCHK] = m;
+      else s_w[w] = m;
+    }
+  } else if (WPS > 1 && lane == 0) {
+    s_w[w] = kZero256;
+  }
+  if constexpr (WPS > 1) {
+    __syncthreads();
+    const int t = (int)threadIdx.x;
+    const int sub = (int)blockIdx.x * (npn::kContractBlock / MCHK) + t;
+    if (t < npn::kContractBlock / MCHK && sub < a.nchm) {
+      u256 m = s_w[WPS * t];
+#pragma unroll
+      for (int k = 1; k < WPS; ++k) m = add256(m, s_w[WPS * t + k]);
+      a.cmass[(size_t)b * a.nchm + sub] = m;
+    }
+  }
 }
 
 // Inverse CDF, one block per sequence, three levels walked by wave 0. (1) The sequence's
@@ -1005,9 +1042,12 @@ __global__ __launch_bounds__(THREADS) void rej_pick_kernel(RejArgs a) {
     }
     u256 gsum = kZero256;
 #pragma unroll
-    for (int k = 0; k < kPickMaxGroup; ++k) gsum = add256(gsum, mv[k]);
+    for (int k = 0; k < kPickMaxGroup; ++k) {
+      if (k >= G) break;
+      gsum = add256(gsum, mv[k]);
+    }
     const u256 incl = wave_incl_scan_u256(gsum);
-    const u256 tot = shfl_u256(incl, 63);
+    const u256 tot = read_lane_u256(incl, 63);
     const u256 target = mul256x32(tot, uniform_fix(a.u_sample[b]));  // need 2^24 C > target
     // a positive total always crosses (U < 2^24)
     const uint64_t hit = __builtin_amdgcn_ballot_w64(gt256(shl24_256(incl), target));
@@ -1015,15 +1055,15 @@ __global__ __launch_bounds__(THREADS) void rej_pick_kernel(RejArgs a) {
       if (lane == 0) s_tok = -1;
     } else {
       const int l = __builtin_ctzll(hit);
-      u256 run = shfl_u256(sub256(incl, gsum), l);  // mass before lane l's group
+      u256 run = read_lane_u256(sub256(incl, gsum), l);  // mass before lane l's group
       int sub = a.nchm - 1;
       u256 before = kZero256;
       bool found = false;
 #pragma unroll
       for (int k = 0; k < kPickMaxGroup; ++k) {
-        const u256 mk = shfl_u256(mv[k], l);
-        const u256 next = add256(run, mk);
-        if (k < G && !found && gt256(shl24_256(next), target)) {
+        if (k >= G) break;
+        const u256 next = add256(run, read_lane_u256(mv[k], l));
+        if (!found && gt256(shl24_256(next), target)) {
           sub = l * G + k;
           before = run;
           found = true;
@@ -1041,7 +1081,7 @@ __global__ __launch_bounds__(THREADS) void rej_pick_kernel(RejArgs a) {
       const uint64_t chit =
           __builtin_amdgcn_ballot_w64(cin && gt256(shl24_256(add256(before, cincl)), target));
       const int cl = chit ? __builtin_ctzll(chit) : 0;
-      const u256 cbefore = add256(before, shfl_u256(sub256(cincl, mc), cl));
+      const u256 cbefore = add256(before, read_lane_u256(sub256(cincl, mc), cl));
       // (3) the chunk's entries
       const int v = (sub * (MCHK / CC) + cl) * CC + lane;
       float pv = NAN, qv = NAN;
@@ -1201,12 +1241,18 @@ void launch_stats(const RejArgs& a, int row0, int rows, hipStream_t s) {
 // the LM-head form.
 template <typename TT>
 int launch_decide_sample(const RejArgs& a, hipStream_t s) {
-  const dim3 mgrid((a.nchm + THREADS / 64 - 1) / (THREADS / 64), a.B);
+  const dim3 mgrid(a.nb, a.B);
+  const bool few = (long)a.nb * a.B <= MASS_WG;
+  auto mass = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, mgrid, dim3(threads), 0, s, a);
+  };
   if (a.inv_temp == 1.0f) {
-    hipLaunchKernelGGL((rej_mass_kernel<true, TT>), mgrid, dim3(THREADS), 0, s, a);
+    if (few) mass(rej_mass_kernel<true, TT, 8>, npn::kContractBlock / 8);
+    else mass(rej_mass_kernel<true, TT, 32>, npn::kContractBlock / 32);
     hipLaunchKernelGGL((rej_pick_kernel<true, TT>), dim3(a.B), dim3(THREADS), 0, s, a);
   } else {
-    hipLaunchKernelGGL((rej_mass_kernel<false, TT>), mgrid, dim3(THREADS), 0, s, a);
+    if (few) mass(rej_mass_kernel<false, TT, 8>, npn::kContractBlock / 8);
+    else mass(rej_mass_kernel<false, TT, 32>, npn::kContractBlock / 32);
     hipLaunchKernelGGL((rej_pick_kernel<false, TT>), dim3(a.B), dim3(THREADS), 0, s, a);
   }
   return npn_launch_status();
