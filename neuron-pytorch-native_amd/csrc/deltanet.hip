@@ -18,6 +18,7 @@
 // split into row parts (the verify kernel below); the workgroup size follows the batch, so
 // small batches still stream the states through many waves.
 #include "npn_common.h"
+#include "npn_internal.h"
 
 namespace {
 
@@ -43,15 +44,16 @@ struct DnArgs {
   int B, T, Hk, Hv;
   int nsplit;  // workgroups per head, each storing 128 / nsplit of the head's columns
   uint16_t* conv_out;  // T == 1: the shifted conv window [B][QKV][3] (nullptr: not written)
+  npn::TokenParts parts;  // B == T == 1: mixed_qkv and z as split-K partials (the PARTS kernel)
 };
 
-// Depthwise causal conv (4 taps, oldest first) + bias + SiLU of channel c over T tokens.
-template <int TMAX>
-__device__ __forceinline__ void conv_channel(const uint16_t* __restrict__ cs,
-                                             const uint16_t* __restrict__ x,
+// Depthwise causal conv (4 taps, oldest first) + bias + SiLU of channel c over T tokens, whose
+// inputs are x(t).
+template <int TMAX, class X>
+__device__ __forceinline__ void conv_channel(const uint16_t* __restrict__ cs, X&& x,
                                              const float* __restrict__ w,
-                                             const float* __restrict__ bias, int c, int QKV,
-                                             int T, float (&y)[TMAX]) {
+                                             const float* __restrict__ bias, int c, int T,
+                                             float (&y)[TMAX]) {
   const float w0 = w[c * 4 + 0], w1 = w[c * 4 + 1], w2 = w[c * 4 + 2], w3 = w[c * 4 + 3];
   const float bc = bias[c];
   float s0 = npn::bf16_to_f32(cs[c * 3 + 0]);
@@ -60,7 +62,7 @@ __device__ __forceinline__ void conv_channel(const uint16_t* __restrict__ cs,
 #pragma unroll
   for (int t = 0; t < TMAX; ++t) {
     if (t < T) {
-      const float xt = npn::bf16_to_f32(x[(size_t)t * QKV + c]);
+      const float xt = npn::bf16_to_f32(x(t));
       y[t] = npn::silu(w0 * s0 + w1 * s1 + w2 * s2 + w3 * xt + bc);
       s0 = s1;
       s1 = s2;
@@ -69,6 +71,23 @@ __device__ __forceinline__ void conv_channel(const uint16_t* __restrict__ cs,
       y[t] = 0.0f;
     }
   }
+}
+
+// Column c of a one-row GEMM from its split-K partials [S][n], summed in slot order and scaled:
+// the bf16 value npn_fp8_matmul writes. Eight loads in flight (past S they repeat slot S - 1).
+__device__ __forceinline__ uint16_t part_value(const float* part, int S, int n,
+                                               const float* scale, int c) {
+  const float sc = scale[c];
+  float acc = 0.f;
+  for (int s0 = 0; s0 < S; s0 += 8) {
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = part[(size_t)min(s0 + j, S - 1) * n + c];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (s0 + j < S) acc += v[j];
+  }
+  return npn::f32_to_bf16(acc * sc);
 }
 
 // Verify kernel: one workgroup of 128 * P threads per (b, h). Wave w holds state columns
@@ -83,8 +102,13 @@ __device__ __forceinline__ void conv_channel(const uint16_t* __restrict__ cs,
 // columns of every checkpoint and output row. The checkpoint stores, which a CU issues at a
 // limited rate, then spread over nsplit times as many CUs; a head's workgroups are heads
 // blocks apart, so with heads % 8 == 0 they share an XCD (and its L2 copy of the state).
-template <int TMAX, int P>
+// PARTS (one token of one sequence): mixed_qkv and z come as the projections' split-K partials,
+// which every workgroup reduces for its own head's channels. As a kernel of its own between the
+// GEMM and this one the reduction took 4.7 to 5.9 us (deltanet::full_fp8, 16/48 heads, graph
+// replays: 31.4 us with it, 28.1 without).
+template <int TMAX, int P, bool PARTS>
 __global__ __launch_bounds__(128 * P) void dn_verify_kernel(DnArgs a) {
+  static_assert(!PARTS || TMAX == 1, "partials of one token");
   constexpr int R = D / P;             // state rows per thread
   constexpr int NT = 128 * P;
   const int heads = a.B * a.Hv;
@@ -111,6 +135,7 @@ __global__ __launch_bounds__(128 * P) void dn_verify_kernel(DnArgs a) {
   __shared__ float s_v[TMAX][D];
   __shared__ float s_o[TMAX][D];
   __shared__ float s_rq[TMAX], s_rk[TMAX], s_ro[TMAX];
+  __shared__ float s_z[PARTS ? D : 1];
   __shared__ float s_decay[TMAX];
   __shared__ float s_beta[TMAX];
   __shared__ float s_red[2][2][P][D];  // [S^T k | S^T q][token parity][row part][column]
@@ -131,12 +156,20 @@ __global__ __launch_bounds__(128 * P) void dn_verify_kernel(DnArgs a) {
   {
     const uint16_t* xb = a.mixed_qkv + (size_t)b * T * QKV;
     const uint16_t* csb = a.conv_state + (size_t)b * QKV * 3;
-    for (int ch = tid; ch < 3 * D; ch += NT) {
+    for (int ch = tid; ch < 3 * D + (PARTS ? cspan : 0); ch += NT) {
       const int which = ch / D, i = ch - which * D;
+      if (PARTS && which == 3) {
+        s_z[i] = npn::bf16_to_f32(
+            part_value(a.parts.pz, a.parts.sz, a.Hv * D, a.parts.zs, h * D + cs0 + i));
+        continue;
+      }
       const int chan = which == 0 ? kh * D + i : (which == 1 ? (a.Hk + kh) * D + i : (2 * a.Hk + h) * D + i);
       float (*dst)[D] = which == 0 ? s_q : (which == 1 ? s_k : s_v);
       float y[TMAX];
-      conv_channel<TMAX>(csb, xb, a.conv_weight, a.conv_bias, chan, QKV, T, y);
+      uint16_t x0 = 0;
+      if constexpr (PARTS) x0 = part_value(a.parts.pq, a.parts.sq, QKV, a.parts.qs, chan);
+      auto x = [&](int t) { return PARTS ? x0 : xb[(size_t)t * QKV + chan]; };
+      conv_channel<TMAX>(csb, x, a.conv_weight, a.conv_bias, chan, T, y);
 #pragma unroll
       for (int t = 0; t < TMAX; ++t) dst[t][i] = y[t];
       // The single-token window shift [cs1, cs2, x] of the channels this workgroup owns: its
@@ -147,7 +180,7 @@ __global__ __launch_bounds__(128 * P) void dn_verify_kernel(DnArgs a) {
         uint16_t* co = a.conv_out + ((size_t)b * QKV + chan) * 3;
         co[0] = cs[1];
         co[1] = cs[2];
-        co[2] = xb[chan];
+        co[2] = x(0);
       }
     }
   }
@@ -239,7 +272,7 @@ __global__ __launch_bounds__(128 * P) void dn_verify_kernel(DnArgs a) {
   for (int idx = tid; idx < T * cspan; idx += NT) {
     const int t = idx / cspan, cc = cs0 + (idx - t * cspan);
     const size_t oi = (((size_t)b * T + t) * a.Hv + h) * D + cc;
-    const float zz = npn::bf16_to_f32(a.z[oi]);
+    const float zz = PARTS ? s_z[cc - cs0] : npn::bf16_to_f32(a.z[oi]);
     a.out[oi] = npn::f32_to_bf16(s_o[t][cc] * s_ro[t] * a.norm_weight[cc] * npn::silu(zz));
   }
 }
@@ -343,15 +376,15 @@ int row_parts(int heads) { return heads < 192 ? 8 : (heads < 1536 ? 4 : 2); }
 // with eight (two workgroups per CU, each computing its whole head).
 int col_splits(int heads) { return heads <= 64 ? 4 : (heads <= 128 ? 2 : 1); }
 
-template <int TMAX>
+template <int TMAX, bool PARTS = false>
 void launch_verify(DnArgs a, hipStream_t s) {
   const int heads = a.B * a.Hv;
   a.nsplit = col_splits(heads);
   const dim3 grid(heads * a.nsplit);
   switch (row_parts(heads)) {
-    case 2: hipLaunchKernelGGL((dn_verify_kernel<TMAX, 2>), grid, dim3(256), 0, s, a); break;
-    case 4: hipLaunchKernelGGL((dn_verify_kernel<TMAX, 4>), grid, dim3(512), 0, s, a); break;
-    default: hipLaunchKernelGGL((dn_verify_kernel<TMAX, 8>), grid, dim3(1024), 0, s, a); break;
+    case 2: hipLaunchKernelGGL((dn_verify_kernel<TMAX, 2, PARTS>), grid, dim3(256), 0, s, a); break;
+    case 4: hipLaunchKernelGGL((dn_verify_kernel<TMAX, 4, PARTS>), grid, dim3(512), 0, s, a); break;
+    default: hipLaunchKernelGGL((dn_verify_kernel<TMAX, 8, PARTS>), grid, dim3(1024), 0, s, a); break;
   }
 }
 
@@ -380,11 +413,32 @@ int verify_checked(const float* state, const int32_t* state_index, int state_T,
   NPN_REQUIRE(NPN_ALIGNED16(state) && NPN_ALIGNED16(ckpt), NPN_ERR_ALIGN);
   DnArgs a{state, state_index, state_T, mixed_qkv, conv_state, conv_weight, conv_bias,
            a_out,  b_out,       z,       A_log,     dt_bias,    norm_weight, ckpt,
-           out,    B,           T,       k_heads,   v_heads,   1,           conv_out};
+           out,    B,           T,       k_heads,   v_heads,   1,           conv_out,
+           {}};
   return verify_impl(a, static_cast<hipStream_t>(stream));
 }
 
 }  // namespace
+
+namespace npn {
+
+int deltanet_token_parts(const float* state, const TokenParts& parts, const uint16_t* conv_state,
+                         const float* conv_weight, const float* conv_bias, const float* a_out,
+                         const float* b_out, const float* A_log, const float* dt_bias,
+                         const float* norm_weight, float* new_state, uint16_t* new_conv_state,
+                         uint16_t* out, int k_heads, int v_heads, hipStream_t stream) {
+  const int st = check_heads(k_heads, v_heads);
+  if (st != NPN_OK) return st;
+  NPN_REQUIRE(NPN_ALIGNED16(state) && NPN_ALIGNED16(new_state), NPN_ERR_ALIGN);
+  const DnArgs a{state, nullptr, 0,      nullptr, conv_state, conv_weight, conv_bias,
+                 a_out, b_out,   nullptr, A_log,  dt_bias,    norm_weight, new_state,
+                 out,   1,       1,       k_heads, v_heads,   1,           new_conv_state,
+                 parts};
+  launch_verify<1, true>(a, stream);
+  return npn_launch_status();
+}
+
+}  // namespace npn
 
 extern "C" int npn_deltanet_verify(const float* state, const int32_t* state_index, int state_T,
                                    const uint16_t* mixed_qkv, const uint16_t* conv_state,

@@ -111,6 +111,76 @@ __device__ __forceinline__ void transpose_dequant(const uint32_t (&d)[8], bf16x8
   }
 }
 
+// Two thin fp32 projections of one row, out_j[n] = (sum_k x[k] * W_j[k][n]) * scale_j[n], W_j
+// [K, n] e4m3fn bytes: the decay and beta inputs of a DeltaNet token (n = Hv). A workgroup of
+// 256 threads takes `per` adjacent columns of one matrix (4 where n allows 4-byte reads, else
+// 1); thread t adds k = t, t + 256, ... in order, then the wave sums (fixed butterfly) and the
+// four waves in order: the same bits every run. They run beside the token's wide projections,
+// in their launch and after them in its grid: first in it, they held back the GEMM's workgroups
+// on their CUs (16/48 heads: 20 us for the launch against 18.2).
+struct ThinArgs {
+  const uint16_t* x;
+  const uint8_t* w[2];
+  const float* scale[2];
+  float* out[2];
+  int K, n, per;
+  __host__ __device__ int blocks() const { return 2 * (n / per); }
+};
+
+template <int PER>
+__device__ __forceinline__ void thin_projection(const ThinArgs& a, int blk, float* part) {
+  const int groups = a.n / PER, j = blk >= groups ? 1 : 0, col = (blk - j * groups) * PER;
+  const uint8_t* w = (j ? a.w[1] : a.w[0]) + col;
+  const int tid = threadIdx.x, lane = tid & 63;
+  // U loads per thread in flight at once (one batch for K = 5120); indices past K are clamped
+  // to K - 1 so the loads need no branch, and their products are not added
+  constexpr int U = 20;
+  float acc[PER] = {};
+  for (int k0 = tid; k0 < a.K; k0 += 256 * U) {
+    uint32_t xv[U], wv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = min(k0 + 256 * u, a.K - 1);
+      xv[u] = a.x[k];
+      if constexpr (PER == 4) wv[u] = *reinterpret_cast<const uint32_t*>(w + (size_t)k * a.n);
+      else wv[u] = w[(size_t)k * a.n];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (k0 + 256 * u >= a.K) continue;
+      const float x = npn::bf16_to_f32(xv[u]);
+      const uint32_t lo = fp8x2_to_bf16x2<false>(wv[u]);
+      acc[0] += x * npn::bf16lo(lo);
+      if constexpr (PER == 4) {
+        const uint32_t hi = fp8x2_to_bf16x2<true>(wv[u]);
+        acc[1] += x * npn::bf16hi(lo);
+        acc[2] += x * npn::bf16lo(hi);
+        acc[3] += x * npn::bf16hi(hi);
+      }
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < PER; ++c) {
+    acc[c] = npn::wave_sum(acc[c]);
+    if (lane == 0) part[(tid >> 6) * PER + c] = acc[c];
+  }
+  __syncthreads();
+  if (tid < PER) {
+    const float s = ((part[tid] + part[PER + tid]) + part[2 * PER + tid]) + part[3 * PER + tid];
+    (j ? a.out[1] : a.out[0])[col + tid] = s * (j ? a.scale[1] : a.scale[0])[col + tid];
+  }
+}
+
+__device__ __forceinline__ void thin_block(const ThinArgs& a, int blk, float* part) {
+  if (a.per == 4) thin_projection<4>(a, blk, part);
+  else thin_projection<1>(a, blk, part);
+}
+
+__global__ __launch_bounds__(256) void fp8_thin_kernel(ThinArgs a) {
+  __shared__ float part[16];
+  thin_block(a, blockIdx.x, part);
+}
+
 struct GemmArgs {
   const uint16_t* x;
   const uint8_t* w;
@@ -126,11 +196,14 @@ struct GemmArgs {
   float* cmax;
   uint64_t* csum;
   float inv_temp;
-  // narrow kernel, tiles1 > 0: a second matrix in the same launch (partials only, no
-  // stream-K): column tiles [0, tiles1) are w's, the rest w2's [K, N2] with partials2
+  // a PAIR launch (one row, partials only): one grid dimension of w's tiles1 tiles x split_k,
+  // then those of a second matrix w2 [K, N2] with its own partials and split, then the thin
+  // projections' workgroups (as tiles x splits in two dimensions, with the shorter split's
+  // spare workgroups leaving at once, the CUs' shares were uneven: 21.8 us against 18.2)
   const uint8_t* w2;
   float* partial2;
   int N2, tiles1, split2;
+  ThinArgs thin;
 };
 
 __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
@@ -178,22 +251,9 @@ __device__ __forceinline__ void wait_tiles(int pend) {
   }
 }
 
-template <int RB, int KG, bool STREAM>
+template <int RB, int KG, bool STREAM, bool PAIR = false>
 __global__ __launch_bounds__(KG * 256, KG) void fp8_gemm_narrow_kernel(GemmArgs ka) {
   static_assert(KG == 1 || !STREAM, "stream-K runs one k group");
-  // A two-matrix launch runs the second matrix's tiles with its pointers and width.
-  GemmArgs a = ka;
-  int tile = blockIdx.x;
-  if (!STREAM && ka.tiles1 > 0) {
-    if (tile >= ka.tiles1) {
-      a.w = ka.w2;
-      a.N = ka.N2;
-      a.partial = ka.partial2;
-      a.split_k = ka.split2;
-      tile -= ka.tiles1;
-    }
-    if ((int)blockIdx.y >= a.split_k) return;
-  }
   constexpr int NTH = KG * 256;
   constexpr int NK = KG * KSTEP;             // k per stage (one k unit)
   constexpr int CH = 4;                      // column slices, one per wave of a k group
@@ -201,12 +261,35 @@ __global__ __launch_bounds__(KG * 256, KG) void fp8_gemm_narrow_kernel(GemmArgs 
   constexpr int WST = NK * NT;               // W stage bytes
   constexpr int XST = 16 * RB * NK * 2;      // x stage bytes, [16 RB rows][32 k] bf16 per group
   constexpr int STAGE = WST + XST;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[NS * STAGE];
+  // A two-matrix launch runs the second matrix's tiles with its pointers and width.
+  GemmArgs a = ka;
+  int tile = blockIdx.x;
+  int sk = blockIdx.y;
+  if constexpr (PAIR) {
+    const int wgs1 = ka.tiles1 * ka.split_k;
+    const int wgs = wgs1 + (ka.N2 + NT - 1) / NT * ka.split2;
+    if (tile >= wgs) {
+      thin_block(ka.thin, tile - wgs, reinterpret_cast<float*>(smem));
+      return;
+    }
+    int tiles = ka.tiles1;
+    if (tile >= wgs1) {
+      a.w = ka.w2;
+      a.N = ka.N2;
+      a.partial = ka.partial2;
+      a.split_k = ka.split2;
+      tile -= wgs1;
+      tiles = (ka.N2 + NT - 1) / NT;
+    }
+    sk = tile / tiles;
+    tile -= sk * tiles;
+  }
   constexpr int WQ = WST / 16 / NTH;         // W DMA instructions (16 bytes) per thread
   constexpr int XW = XST / 16 / 64;          // waves that move x, one 16-byte DMA per lane
   static_assert(WQ * 16 * NTH == WST && XW * 64 * 16 == XST && XW <= NTH / 64,
                 "whole DMA instructions per stage");
   static_assert(KG == 1 || NS * STAGE >= RB * CB * 256 * 16, "the ring holds a group's sums");
-  __shared__ __attribute__((aligned(16))) uint8_t smem[NS * STAGE];
 
   const int m_pass = blockIdx.z * 16 * RB;
   const int tid = threadIdx.x;
@@ -338,7 +421,7 @@ __global__ __launch_bounds__(KG * 256, KG) void fp8_gemm_narrow_kernel(GemmArgs 
     lo = (int)(u0 - (long)tile * nku);
     hi = (int)min(u1 - (long)tile * nku, (long)nku);
   } else {  // the first nku % split_k splits take a unit more
-    const int sk = blockIdx.y, per = nku / a.split_k, more = nku - per * a.split_k;
+    const int per = nku / a.split_k, more = nku - per * a.split_k;
     lo = per * sk + min(sk, more);
     hi = lo + per + (sk < more ? 1 : 0);
   }
@@ -352,7 +435,7 @@ __global__ __launch_bounds__(KG * 256, KG) void fp8_gemm_narrow_kernel(GemmArgs 
     if (!partials) break;
     if (kg != 0) return;
     if constexpr (!STREAM) {
-      store_partial(blockIdx.y, tile * NT, acc, false);
+      store_partial(sk, tile * NT, acc, false);
       return;
     } else {
       const long tb = (long)tile * nku;
@@ -1596,108 +1679,35 @@ int launch_gemm(const GemmPlan& p, const uint16_t* x, const int8_t* w, const flo
   return npn_launch_status();
 }
 
-// The split-K partials of two GEMMs of the same x ([M, K], M <= 16) in one narrow launch, W1
-// [K, N1] into p1 [S1][M][N1] and W2 [K, N2] into p2 [S2][M][N2]: the same tiles, k ranges and
-// sums as two launches of their plans, which must be narrow tiles x split grids of one pass.
-// Returns false (nothing launched) when they are not.
-bool launch_gemm_pair_partials(const uint16_t* x, const int8_t* w1, float* p1, int N1,
-                               const int8_t* w2, float* p2, int N2, int M, int K,
-                               hipStream_t s) {
-  const GemmPlan a = plan(M, K, N1), b = plan(M, K, N2);
-  if (M > 16 || a.sk_wg > 0 || b.sk_wg > 0) return false;
+// The split-K partials of two GEMMs of the same row x [K] in one narrow launch, W1 [K, N1] into
+// p1 [S1][N1] and W2 [K, N2] into p2 [S2][N2], and the thin projections beside them: the same
+// tiles, k ranges and sums as launches of their own. Stream-K plans do take their own launches.
+int launch_token_projections(const uint16_t* x, const int8_t* w1, float* p1, int N1,
+                             const int8_t* w2, float* p2, int N2, int K, const ThinArgs& thin,
+                             hipStream_t s) {
+  const GemmPlan a = plan(1, K, N1), b = plan(1, K, N2);
+  if (a.sk_wg > 0 || b.sk_wg > 0) {
+    int st = launch_gemm(a, x, w1, nullptr, nullptr, p1, 1, K, N1, 1, false, s);
+    if (st == NPN_OK) st = launch_gemm(b, x, w2, nullptr, nullptr, p2, 1, K, N2, 1, false, s);
+    if (st != NPN_OK) return st;
+    hipLaunchKernelGGL(fp8_thin_kernel, dim3(thin.blocks()), dim3(256), 0, s, thin);
+    return npn_launch_status();
+  }
   const int t1 = (N1 + NT - 1) / NT, t2 = (N2 + NT - 1) / NT;
-  GemmArgs ga{x, reinterpret_cast<const uint8_t*>(w1), nullptr, nullptr, p1, M, K, N1,
+  GemmArgs ga{x, reinterpret_cast<const uint8_t*>(w1), nullptr, nullptr, p1, 1, K, N1,
               a.split_k, 1, nullptr, nullptr, 0, nullptr, nullptr, 1.0f,
-              reinterpret_cast<const uint8_t*>(w2), p2, N2, t1, b.split_k};
-  launch_narrow(ga, a.mt, false, dim3(t1 + t2, std::max(a.split_k, b.split_k), 1), s);
-  return true;
+              reinterpret_cast<const uint8_t*>(w2), p2, N2, t1, b.split_k, thin};
+  hipLaunchKernelGGL((fp8_gemm_narrow_kernel<1, 1, false, true>),
+                     dim3(thin.blocks() + t1 * a.split_k + t2 * b.split_k), dim3(256), 0, s, ga);
+  return npn_launch_status();
 }
 
-// The end of deltanet::full_fp8's in-projections, in one launch after the two GEMMs:
-//  - blocks [0, nq): the qkv GEMM's split-K partials reduced in slot order and scaled into
-//    bf16 mixed_qkv (the values npn_fp8_matmul writes; a sum of one slot is that slot), and the
-//    new conv window [conv_state[:, 1:] | mixed_qkv];
-//  - blocks [nq, nq + nz): the same reduction for z;
-//  - the last 2 * hv blocks: the thin in_proj_a / in_proj_b projections in float32, column n
-//    of matrix j per block: out_j[n] = (sum_k x[k] * W_j[k][n]) * scale_j[n], W_j [K, hv]
-//    e4m3fn bytes (rows hv bytes apart: the two matrices are a few hundred KB, read once from
-//    HBM and then from L2). Thread t adds k = t, t + 256, ... in order, then the wave sums
-//    (fixed butterfly) and the four waves in order: the same bits every run.
-struct InprojFinishArgs {
-  const float* pq;          // [sq][qkv] partials of x . qkv_w
-  const float* qs;
-  uint16_t* mixed;
-  const uint16_t* conv_in;  // [qkv][3]
-  uint16_t* conv_out;
-  const float* pz;          // [sz][zn] partials of x . z_w
-  const float* zs;
-  uint16_t* z;
-  const uint16_t* x;
-  const uint8_t* wa;
-  const float* sa;
-  float* a;
-  const uint8_t* wb;
-  const float* sb;
-  float* b;
-  int sq, qkv, sz, zn, K, hv;
-};
-
-__global__ __launch_bounds__(256) void dn_fp8_inproj_finish_kernel(InprojFinishArgs p) {
-  const int nq = (p.qkv + 255) / 256, nz = (p.zn + 255) / 256;
-  const int blk = blockIdx.x;
-  if (blk < nq + nz) {
-    const bool isq = blk < nq;
-    const int n = isq ? p.qkv : p.zn;
-    const int i = (isq ? blk : blk - nq) * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float* P = isq ? p.pq : p.pz;
-    const int S = isq ? p.sq : p.sz;
-    float acc = P[i];
-    for (int k = 1; k < S; ++k) acc += P[(size_t)k * n + i];
-    const uint16_t v = npn::f32_to_bf16(acc * (isq ? p.qs : p.zs)[i]);
-    if (isq) {
-      p.mixed[i] = v;
-      p.conv_out[3 * i] = p.conv_in[3 * i + 1];
-      p.conv_out[3 * i + 1] = p.conv_in[3 * i + 2];
-      p.conv_out[3 * i + 2] = v;
-    } else {
-      p.z[i] = v;
-    }
-    return;
-  }
-  const int j = (blk - nq - nz) / p.hv, col = (blk - nq - nz) - j * p.hv;
-  const uint8_t* w = j ? p.wb : p.wa;
-  // U loads per thread in flight at once (one batch for HIDDEN = 5120); indices past K are
-  // clamped to K - 1 so the loads need no branch, and their products are not added
-  constexpr int U = 20;
-  float acc = 0.f;
-  for (int k0 = threadIdx.x; k0 < p.K; k0 += 256 * U) {
-    float xv[U], wv[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = min(k0 + 256 * u, p.K - 1);
-      xv[u] = npn::bf16_to_f32(p.x[k]);
-      wv[u] = npn::bf16lo(fp8x2_to_bf16x2<false>(w[(size_t)k * p.hv + col]));
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (k0 + 256 * u < p.K) acc += xv[u] * wv[u];
-  }
-  acc = npn::wave_sum(acc);
-  __shared__ float part[4];
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const float sc = (j ? p.sb : p.sa)[col];
-    (j ? p.b : p.a)[col] = (((part[0] + part[1]) + part[2]) + part[3]) * sc;
-  }
-}
-
-// Workspace of npn_deltanet_full_fp8, 256-byte aligned regions: mixed_qkv [QKV] bf16, z
-// [Hv * 128] bf16, a_out and b_out [Hv] f32, then the split-K partials of the qkv and z GEMMs
-// ([S][N] f32 each, S from the GEMM plan for one row).
+// Workspace of npn_deltanet_full_fp8, 256-byte aligned regions: room for mixed_qkv [QKV] and z
+// [Hv * 128] as bf16 (no kernel writes them; the size stays what callers have allocated), a_out
+// and b_out [Hv] f32, then the split-K partials of the qkv and z GEMMs ([S][N] f32 each, S from
+// the GEMM plan for one row).
 struct FullFp8Layout {
-  size_t z, a, b, pq, pz, total;
+  size_t a, b, pq, pz, total;
   int sq, sz;
 };
 
@@ -1706,8 +1716,7 @@ FullFp8Layout full_fp8_layout(int H, int qkv, int hv) {
   FullFp8Layout l;
   l.sq = plan(1, H, qkv).split_k;
   l.sz = plan(1, H, hv * 128).split_k;
-  l.z = up((size_t)qkv * 2);
-  l.a = l.z + up((size_t)hv * 128 * 2);
+  l.a = up((size_t)qkv * 2) + up((size_t)hv * 128 * 2);
   l.b = l.a + up((size_t)hv * 4);
   l.pq = l.b + up((size_t)hv * 4);
   l.pz = l.pq + up((size_t)l.sq * qkv * 4);
@@ -1902,11 +1911,11 @@ int fp8_matmul_chunk_stats(const uint16_t* x, const int8_t* w, const float* scal
 }  // namespace npn
 
 // deltanet::full_fp8: the four in-projections of one decode token, then the token step of
-// deltanet::full on their outputs. Three launches: the qkv and z GEMMs writing split-K partials
-// (the plans of npn_fp8_matmul for one row, both in one narrow launch where the two plans share
-// their split-K factor, else one launch each), the finishing kernel above (mixed_qkv and z as
-// npn_fp8_matmul's bf16 outputs, the new conv window, a_out and b_out in float32, not rounded),
-// and the DeltaNet token step (npn_deltanet_verify with T = 1).
+// deltanet::full on their outputs. Two launches: the qkv and z GEMMs writing split-K partials
+// (the plans of npn_fp8_matmul for one row) with a_out and b_out in float32, not rounded,
+// beside them, and the DeltaNet token step, which reduces the partials to mixed_qkv and z as
+// npn_fp8_matmul's bf16 outputs and shifts the conv window. (Stream-K plans, from 14080
+// columns on, make four launches of the first.)
 extern "C" size_t npn_deltanet_full_fp8_workspace_size(int hidden, int k_heads, int v_heads) {
   if (!full_fp8_heads_ok(k_heads, v_heads)) return 0;
   const int qkv = (2 * k_heads + v_heads) * 128;
@@ -1944,28 +1953,16 @@ extern "C" int npn_deltanet_full_fp8(
   hipStream_t s = static_cast<hipStream_t>(stream);
   float* pq = reinterpret_cast<float*>(ws + l.pq);
   float* pz = reinterpret_cast<float*>(ws + l.pz);
-  // both GEMMs in one launch where their plans allow (the same partials as two launches)
-  int st = NPN_OK;
-  if (launch_gemm_pair_partials(x, qkv_w, pq, qkv, z_w, pz, zn, 1, hidden, s)) {
-    st = npn_launch_status();
-  } else {
-    st = launch_gemm(plan(1, hidden, qkv), x, qkv_w, nullptr, nullptr, pq, 1, hidden, qkv, 1,
-                     false, s);
-    if (st == NPN_OK)
-      st = launch_gemm(plan(1, hidden, zn), x, z_w, nullptr, nullptr, pz, 1, hidden, zn, 1,
-                       false, s);
-  }
+  float* ab[2] = {reinterpret_cast<float*>(ws + l.a), reinterpret_cast<float*>(ws + l.b)};
+  const bool by4 = v_heads % 4 == 0 && ((reinterpret_cast<uintptr_t>(a_w) |
+                                         reinterpret_cast<uintptr_t>(b_w)) & 3) == 0;
+  const ThinArgs thin{x, {reinterpret_cast<const uint8_t*>(a_w),
+                          reinterpret_cast<const uint8_t*>(b_w)},
+                      {a_s, b_s}, {ab[0], ab[1]}, hidden, v_heads, by4 ? 4 : 1};
+  const int st = launch_token_projections(x, qkv_w, pq, qkv, z_w, pz, zn, hidden, thin, s);
   if (st != NPN_OK) return st;
-  InprojFinishArgs fa{pq, qkv_s, reinterpret_cast<uint16_t*>(ws), conv_state, new_conv_state,
-                      pz, z_s, reinterpret_cast<uint16_t*>(ws + l.z), x,
-                      reinterpret_cast<const uint8_t*>(a_w), a_s, reinterpret_cast<float*>(ws + l.a),
-                      reinterpret_cast<const uint8_t*>(b_w), b_s, reinterpret_cast<float*>(ws + l.b),
-                      l.sq, qkv, l.sz, zn, hidden, v_heads};
-  const int blocks = (qkv + 255) / 256 + (zn + 255) / 256 + 2 * v_heads;
-  hipLaunchKernelGGL(dn_fp8_inproj_finish_kernel, dim3(blocks), dim3(256), 0, s, fa);
-  st = npn_launch_status();
-  if (st != NPN_OK) return st;
-  return npn_deltanet_verify(state, nullptr, 0, fa.mixed, conv_state, conv_weight, conv_bias,
-                             fa.a, fa.b, fa.z, A_log, dt_bias, norm_weight, new_state, out, 1, 1,
-                             k_heads, v_heads, stream);
+  return npn::deltanet_token_parts(state, npn::TokenParts{pq, qkv_s, pz, z_s, l.sq, l.sz},
+                                   conv_state, conv_weight, conv_bias, ab[0], ab[1], A_log,
+                                   dt_bias, norm_weight, new_state, new_conv_state, out, k_heads,
+                                   v_heads, s);
 }

@@ -27,4 +27,21 @@ bool fp8_matmul_stats_pass_cheaper(int M, int K, int N);
 int fp8_matmul_unsplit(const uint16_t* x, const int8_t* w, const float* scale, uint16_t* out,
                        int M, int K, int N, hipStream_t stream);
 
+// The qkv and z projections of one token as fp32 split-K partials: pq [sq][QKV] and pz
+// [sz][Hv * 128] with the per-column scales qs and zs.
+struct TokenParts {
+  const float* pq;
+  const float* qs;
+  const float* pz;
+  const float* zs;
+  int sq, sz;
+};
+// npn_deltanet_full_batched's step of one sequence (deltanet.hip) on those partials, reduced to
+// the bf16 values that npn_fp8_matmul writes. new_conv_state must not overlap conv_state.
+int deltanet_token_parts(const float* state, const TokenParts& parts, const uint16_t* conv_state,
+                         const float* conv_weight, const float* conv_bias, const float* a_out,
+                         const float* b_out, const float* A_log, const float* dt_bias,
+                         const float* norm_weight, float* new_state, uint16_t* new_conv_state,
+                         uint16_t* out, int k_heads, int v_heads, hipStream_t stream);
+
 }  // namespace npn

@@ -16,7 +16,7 @@ import pytest
 import torch
 
 from oracle import deltanet as od
-from _util import BF16_U, assert_rel_close, bits, fp8_weights
+from _util import BF16_U, BF16_ULP, assert_rel_close, bits, fp8_weights
 
 pytestmark = pytest.mark.gpu
 
@@ -89,6 +89,34 @@ def test_full_fp8_matches_oracle(ops, hk, hv, seed):
     # the oracle's mixed_qkv (float64 products) agrees up to rare one-ulp bf16 flips
     assert np.mean(bits(ncs) == cs_ref) > 0.99
     assert torch.equal(ns, ns2) and torch.equal(ncs, ncs2) and torch.equal(out, out2)
+
+
+# v heads that allow 4-byte reads of the thin projections' rows and ones that don't, and qkv and
+# z grids of unequal splits
+@pytest.mark.parametrize("hk,hv", [(1, 3), (5, 15), (8, 24), (1, 1)])
+def test_full_fp8_head_counts(ops, hk, hv):
+    """State against the oracle; the gated output against the token step on fp8::matmul's
+    projections (a and b in float64): both round the same z to bf16, so only the output's own
+    rounding can differ. The oracle rounds z elsewhere, and z's and the output's rounding, 2^-8 /
+    sqrt(3) rms of a binade's bottom each, make 2e-3 of a norm over one head's 128 values."""
+    d = _inputs(hk, hv, 20 + hv)
+    args = _gpu_args(d)
+    ns, ncs, out = ops.deltanet.full_fp8(*args)
+    mixed = ops.fp8.matmul(args[0], args[8], args[9])
+    z = ops.fp8.matmul(args[0], args[10], args[11])
+    a, b = ((args[0].double() @ args[i].view(torch.float8_e4m3fn).double()
+             * args[i + 1].double().reshape(1, hv)).float() for i in (12, 14))
+    ns2, ncs2, out2 = ops.deltanet.full_batched(
+        args[1], mixed.reshape(-1), args[2], args[3], args[4], a.reshape(-1), b.reshape(-1),
+        z.reshape(hv, D), *args[5:8])
+    torch.cuda.synchronize()
+    s_ref, _, _ = _oracle(d, hk, hv)
+    assert_rel_close(ns.cpu().double().numpy().reshape(s_ref.shape), s_ref, name="state")
+    assert_rel_close(ns.cpu().double().numpy(), ns2.cpu().double().numpy(), tol=1e-5,
+                     name="state, fp32 sums of 5120 products in another order")
+    assert_rel_close(out.float().cpu().double().numpy(), out2.float().cpu().double().numpy(),
+                     out_unit=BF16_ULP, name="out")
+    assert torch.equal(ncs.view(torch.int16), ncs2.view(torch.int16))
 
 
 def test_full_fp8_rejects_bad_arguments(ops):
