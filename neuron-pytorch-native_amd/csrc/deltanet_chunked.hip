@@ -20,11 +20,11 @@
 // - dn_chunk_prep_kernel, persistent workgroups over all (head, chunk) items at once:
 //   everything that does not depend on the state -- the per-token scales (row norms folded
 //   with e^g_cum), A, T and the intra-chunk attention -- into a workspace record per item.
-// - dn_chunk_scan_kernel, one workgroup of 8 waves per (head, 32-column block of V), chunk
-//   after chunk: only the products with the state. The columns of the state evolve
-//   independently, so the 4 blocks of a head run side by side, each holding its 128 x 32
-//   block in registers (and its split in LDS). The 4 workgroups of a head are placed on one
-//   XCD so that they share its L2 for the head's q, k and records.
+// - dn_chunk_scan_kernel, one workgroup of 8 waves per (head, block of 32 columns of V, or 16
+//   up to 32 heads), chunk after chunk: only the products with the state. The columns of the
+//   state evolve independently, so the blocks of a head run side by side, each holding its
+//   part of the state in registers (and its split in LDS). The workgroups of a head are placed
+//   on one XCD so that they share its L2 for the head's q, k and records.
 //
 // Products. Matrix products over the 128 k indices or the 64 tokens of a chunk take split
 // operands: x = hi + lo with hi = bf16(x), lo = bf16(x - hi), and a product of two split
@@ -42,7 +42,6 @@ namespace {
 
 constexpr int CH = 64;                  // tokens per chunk
 constexpr int D = 128;                  // k and v head dims
-constexpr int NCB = 4;                  // 32-column blocks of V per head
 constexpr int MS = CH + 4;              // LDS row stride of the prep's fp32 A and T
 constexpr float kNormEps = 1e-6f;
 constexpr float kQScale = 0.08838834764831845f;  // 1/sqrt(128)
@@ -452,6 +451,20 @@ struct ScanSmem {
 // The wave also owns the state tiles S[16 (P0 + p) .. + 15][16 J .. + 15] of the block's 32
 // columns (p = 0, 1; P0 = 2 ((w >> 1) & 3)) in fp32 registers for the whole prompt.
 
+// Z rows of block I from X (transposed tiles): beta (v - sk1 X), split into zh / zl.
+__device__ __forceinline__ void scan_z(ScanSmem& sm, int I, int J, f32x4 x) {
+  const int lane = threadIdx.x & 63, g4 = lane >> 4, c = lane & 15;
+  const int i = 16 * I + c, zo = i * ZB + 16 * J + 4 * g4;
+  const float4 v = ld4(sm.vr + i * VS + 16 * J + 4 * g4);
+  const float4 sc = sm.sc[i];
+  bf16x4 zh, zl;
+  split4(make_float4(sc.w * (v.x - sc.y * x[0]), sc.w * (v.y - sc.y * x[1]),
+                     sc.w * (v.z - sc.y * x[2]), sc.w * (v.w - sc.y * x[3])),
+         zh, zl);
+  *reinterpret_cast<bf16x4*>(sm.zh + zo) = zh;
+  *reinterpret_cast<bf16x4*>(sm.zl + zo) = zl;
+}
+
 // Pa: X = (raw k) S and O = (raw q) S for rows of block I (split products over the 128 k
 // indices, step st covering 32 st + 8 g .. + 7 for lane group g), formed as transposed tiles
 // (S^T as the A operand) so that x[r], o[r] hold token 16 I + c, column 16 J + 4 g + r: a
@@ -486,16 +499,36 @@ __device__ __forceinline__ void scan_state_products(ScanSmem& sm, int I, int J, 
     x = mfma3(sh, sl, kh, kl, x);
     o = mfma3(sh, sl, qh, ql, o);
   }
-  const int i = 16 * I + c, zo = i * ZB + 16 * J + 4 * g4;
-  const float4 v = ld4(sm.vr + i * VS + 16 * J + 4 * g4);
-  const float4 sc = sm.sc[i];
-  bf16x4 zh, zl;
-  split4(make_float4(sc.w * (v.x - sc.y * x[0]), sc.w * (v.y - sc.y * x[1]),
-                     sc.w * (v.z - sc.y * x[2]), sc.w * (v.w - sc.y * x[3])),
-         zh, zl);
-  *reinterpret_cast<bf16x4*>(sm.zh + zo) = zh;
-  *reinterpret_cast<bf16x4*>(sm.zl + zo) = zl;
-  o *= sc.x;
+  scan_z(sm, I, J, x);
+  o *= sm.sc[16 * I + c].x;
+}
+
+// Pa of the 16-column form: one of the two products, S^T rows against the rows of block I of
+// `hi` / `lo` (k or q), as a transposed tile.
+template <typename Pre>
+__device__ __forceinline__ f32x4 scan_state_product(ScanSmem& sm, const __bf16* hi,
+                                                    const __bf16* lo, int I, Pre&& pre) {
+  const int lane = threadIdx.x & 63, g4 = lane >> 4, c = lane & 15;
+  f32x4 x = zero4();
+  const int rr = 16 * I + c, so = c * RB + 8 * g4;
+  int ro = qk_idx(rr, 8 * g4);
+  bf16x8 nrh = ld8(hi + ro), nrl = ld8(lo + ro), nsh = ld8(sm.sh + so), nsl = ld8(sm.sl + so);
+#pragma unroll
+  for (int st = 0; st < 4; ++st) {
+    const bf16x8 rh = nrh, rl = nrl, sh = nsh, sl = nsl;
+    if (st < 3) {
+      const int d = 32 * (st + 1);
+      ro = qk_idx(rr, d + 8 * g4);
+      nrh = ld8(hi + ro);
+      nrl = ld8(lo + ro);
+      nsh = ld8(sm.sh + so + d);
+      nsl = ld8(sm.sl + so + d);
+    }
+    pre(st);
+    __builtin_amdgcn_sched_barrier(0);
+    x = mfma3(sh, sl, rh, rl, x);
+  }
+  return x;
 }
 
 // acc += T Z for rows of block I over the tokens below 32 ceil((I + 1) / 2) (T is zero above
@@ -540,21 +573,26 @@ __device__ __forceinline__ void scan_vnew(ScanSmem& sm, int I, int J) {
 // registers in Pb: the wave's intra rows (A of the output product, tokens 32 st + 8 g .. + 7;
 // blocks above the diagonal are zero), k's token columns for state tiles P0 + p (B of the
 // state update, read transposed) and e^tot.
+template <int NP>
 struct PcOps {
   bf16x8 ih[2], il[2];
-  bf16x8 kh[2][2], kl[2][2];
+  bf16x8 kh[2][NP], kl[2][NP];
   float et;
 };
-__device__ __forceinline__ void scan_pc_loads(ScanSmem& sm, int I, int P0, PcOps& op) {
+template <int NP>
+__device__ __forceinline__ void scan_pc_loads(ScanSmem& sm, int I, int P0, bool out,
+                                              PcOps<NP>& op) {
   const int lane = threadIdx.x & 63, g4 = lane >> 4, c = lane & 15;
   const int ao = (16 * I + c) * VB + 8 * g4;
 #pragma unroll
   for (int st = 0; st < 2; ++st) {
-    op.ih[st] = ld8(sm.ih + ao + 32 * st);
-    op.il[st] = ld8(sm.il + ao + 32 * st);
+    if (out) {
+      op.ih[st] = ld8(sm.ih + ao + 32 * st);
+      op.il[st] = ld8(sm.il + ao + 32 * st);
+    }
     const int r0 = 32 * st + 8 * g4 + (c >> 2);
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
+    for (int p = 0; p < NP; ++p) {
       const int e = 16 * (P0 + p) + 4 * (c & 3);
       const int b0 = qk_idx(r0, e), b1 = qk_idx(r0 + 4, e);
       op.kh[st][p] = pack8(lds_tr16(sm.kh + b0), lds_tr16(sm.kh + b1));
@@ -567,8 +605,8 @@ __device__ __forceinline__ void scan_pc_loads(ScanSmem& sm, int I, int P0, PcOps
 // Pc: out rows of block I = O + intra v_new (over the tokens below 32 ceil((I + 1) / 2)), a
 // transposed tile like O (v_new^T rows as the A operand, intra rows as the B operand), written
 // where the token exists.
-template <int NST>
-__device__ __forceinline__ void out_tile(ScanSmem& sm, int J, const PcOps& op, f32x4& o) {
+template <int NST, int NP>
+__device__ __forceinline__ void out_tile(ScanSmem& sm, int J, const PcOps<NP>& op, f32x4& o) {
   const int lane = threadIdx.x & 63, g4 = lane >> 4, c = lane & 15;
   const int bo = (16 * J + c) * VB + 8 * g4;
   bf16x8 bh[NST], bl[NST];
@@ -581,8 +619,9 @@ __device__ __forceinline__ void out_tile(ScanSmem& sm, int J, const PcOps& op, f
 #pragma unroll
   for (int st = 0; st < NST; ++st) o = mfma3(bh[st], bl[st], op.ih[st], op.il[st], o);
 }
+template <int NP>
 __device__ __forceinline__ void scan_out(ScanSmem& sm, float* orow, int I, int J, f32x4 o,
-                                         int nvalid, const PcOps& op) {
+                                         int nvalid, const PcOps<NP>& op) {
   const int lane = threadIdx.x & 63, g4 = lane >> 4, c = lane & 15;
   if (I < 2) out_tile<1>(sm, J, op, o);
   else out_tile<2>(sm, J, op, o);
@@ -597,8 +636,9 @@ __device__ __forceinline__ void scan_out(ScanSmem& sm, float* orow, int I, int J
 // 32 st + 8 g .. + 7: the A operand k's token columns from op, the B operand from vsh / vsl
 // rows), then the split of S' to LDS, where a lane's 4 values are consecutive k indices of one
 // S^T row (one 8-byte store per half and tile).
-__device__ __forceinline__ void scan_state_update(ScanSmem& sm, int J, int P0, f32x4 (&s)[2],
-                                                  const PcOps& op) {
+template <int NP>
+__device__ __forceinline__ void scan_state_update(ScanSmem& sm, int J, int P0, f32x4 (&s)[NP],
+                                                  const PcOps<NP>& op) {
   const int lane = threadIdx.x & 63, g4 = lane >> 4, c = lane & 15;
   bf16x8 ah[2], al[2];
 #pragma unroll
@@ -608,14 +648,14 @@ __device__ __forceinline__ void scan_state_update(ScanSmem& sm, int J, int P0, f
     al[st] = ld8(sm.vsl + ao);
   }
 #pragma unroll
-  for (int p = 0; p < 2; ++p) s[p] *= op.et;
+  for (int p = 0; p < NP; ++p) s[p] *= op.et;
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int st = 0; st < 2; ++st)
 #pragma unroll
-    for (int p = 0; p < 2; ++p) s[p] = mfma3(op.kh[st][p], op.kl[st][p], ah[st], al[st], s[p]);
+    for (int p = 0; p < NP; ++p) s[p] = mfma3(op.kh[st][p], op.kl[st][p], ah[st], al[st], s[p]);
 #pragma unroll
-  for (int p = 0; p < 2; ++p) {
+  for (int p = 0; p < NP; ++p) {
     const int o = (16 * J + c) * RB + 16 * (P0 + p) + 4 * g4;
     bf16x4 h, l;
     split4(make_float4(s[p][0], s[p][1], s[p][2], s[p][3]), h, l);
@@ -626,25 +666,35 @@ __device__ __forceinline__ void scan_state_update(ScanSmem& sm, int J, int P0, f
 
 constexpr int kScanThreads = 512;
 
+// NJ = 2: blocks of 32 columns, as described above. NJ = 1: blocks of 16 columns, for few heads:
+// twice the workgroups, each with half the products, and the time of a chunk is the chain of
+// one workgroup (12 heads x 1000 tokens on 48 CUs: 3.2 us a chunk against 2.5 on 96; the call 63.5 -> 52.3).
+// There waves 0..3 form X, Z and v_new of row block 3 - w, waves 4..7 O and out of row block
+// w - 4, and every wave owns one state tile, P0 = w. Every element's products and sums are the
+// same in both forms, so the results are the same bits.
+template <int NJ>
 __global__ __launch_bounds__(kScanThreads, 1) void dn_chunk_scan_kernel(ScanArgs a) {
   __shared__ __attribute__((aligned(16))) ScanSmem sm;
-  // workgroup L runs on XCD L % 8: the 4 column blocks of head h all get XCD h % 8
+  constexpr int NC = 16 * NJ, NCB = D / NC, NP = NJ;  // columns, blocks per head, state tiles
+  // workgroup L runs on XCD L % 8: the NCB column blocks of head h all get XCD h % 8
   const int L = blockIdx.x, grp = L / (8 * NCB), rem = L % (8 * NCB);
   const int cb = rem >> 3, h = 8 * grp + (rem & 7);
   if (h >= a.Hv) return;
   const int tid = threadIdx.x, lane = tid & 63, g4 = lane >> 4, c = lane & 15;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int J = wv & 1;
-  const int I = wv < 4 ? 3 - ((wv >> 1) & 1) : (wv >> 1) & 1;
-  const int P0 = 2 * ((wv >> 1) & 3);
+  const int J = NJ == 2 ? wv & 1 : 0;
+  const int I = NJ == 2 ? (wv < 4 ? 3 - ((wv >> 1) & 1) : (wv >> 1) & 1)
+                        : (wv < 4 ? 3 - wv : wv - 4);
+  const int P0 = NJ == 2 ? 2 * ((wv >> 1) & 3) : wv;
+  const bool forms_x = NJ == 2 || wv < 4, forms_o = NJ == 2 || wv >= 4;
   const int S = a.S;
   const size_t row0 = (size_t)h * S;
-  const int c0 = 32 * cb;
+  const int c0 = NC * cb;
 
   // this wave's state tiles: S[16 (P0 + p) + 4 g + r][c0 + 16 J + c] in s[p][r], and their split
-  f32x4 s[2];
+  f32x4 s[NP];
 #pragma unroll
-  for (int p = 0; p < 2; ++p) {
+  for (int p = 0; p < NP; ++p) {
     const float* src = a.state + ((size_t)h * D + 16 * (P0 + p) + 4 * g4) * D + c0 + 16 * J + c;
 #pragma unroll
     for (int r = 0; r < 4; ++r) s[p][r] = src[r * D];
@@ -670,7 +720,9 @@ __global__ __launch_bounds__(kScanThreads, 1) void dn_chunk_scan_kernel(ScanArgs
   float4 psc = make_float4(0.f, 0.f, 0.f, 0.f);
   float pet = 0.f;
   const int qk_off = (tid >> 5) * (D * 4) + (tid & 31) * 16;        // + 8192 j
-  const int v_off = (tid >> 3) * (D * 4) + (c0 + 4 * (tid & 7)) * 4;
+  // (16 columns: the other half's reads fall past the descriptor and touch nothing)
+  const int v_off = NJ == 2 || (tid & 7) < 4 ? (tid >> 3) * (D * 4) + (c0 + 4 * (tid & 7)) * 4
+                                             : 0x7FFFFFF0;
   auto fetch_part = [&](int ci, int part) {
     const int t0 = ci * CH;
     const int rest = (S - t0) * (D * 4);
@@ -724,7 +776,7 @@ __global__ __launch_bounds__(kScanThreads, 1) void dn_chunk_scan_kernel(ScanArgs
   store_v_t_sc();
   store_k_intra();
   f32x4 o;
-  PcOps op;
+  PcOps<NP> op;
   for (int ci = 0; ci < a.nch; ++ci) {
     const int t0 = ci * CH;
     // the next chunk's reads (unconditional, so that no branch forces an early wait: the last
@@ -735,23 +787,30 @@ __global__ __launch_bounds__(kScanThreads, 1) void dn_chunk_scan_kernel(ScanArgs
       for (int d = 0; d < 3; ++d) fetch_part(nx, 3 * st + d);
     };
     __syncthreads();
-    scan_state_products(sm, I, J, o, pre_a);
+    if constexpr (NJ == 2) {
+      scan_state_products(sm, I, J, o, pre_a);
+    } else {
+      const f32x4 x = scan_state_product(sm, forms_x ? sm.kh : sm.qh, forms_x ? sm.kl : sm.ql, I,
+                                         pre_a);
+      if (forms_x) scan_z(sm, I, J, x);
+      else o = x * sm.sc[16 * I + c].x;
+    }
     __syncthreads();
     fetch_part(nx, 12);
     fetch_part(nx, 13);
-    scan_vnew(sm, I, J);
+    if (forms_x) scan_vnew(sm, I, J);
     // after v_new's operand reads (a wave's LDS requests return in order): frees k, intra and
     // e^tot for the next chunk's stores in Pc
-    scan_pc_loads(sm, I, P0, op);
+    scan_pc_loads(sm, I, P0, forms_o, op);
     store_split(pq, sm.qh, sm.ql);  // q of this chunk was last read in Pa
     __syncthreads();
     scan_state_update(sm, J, P0, s, op);  // first: the next chunk waits on its split of S
-    scan_out(sm, a.out + (row0 + t0) * D + c0, I, J, o, min(CH, S - t0), op);
+    if (forms_o) scan_out(sm, a.out + (row0 + t0) * D + c0, I, J, o, min(CH, S - t0), op);
     store_v_t_sc();  // v, T and the scales were last read in Pa / Pb
     store_k_intra();  // k, intra and e^tot of this chunk were last read in Pa / Pb
   }
 #pragma unroll
-  for (int p = 0; p < 2; ++p) {
+  for (int p = 0; p < NP; ++p) {
     float* dst = a.new_state + ((size_t)h * D + 16 * (P0 + p) + 4 * g4) * D + c0 + 16 * J + c;
 #pragma unroll
     for (int r = 0; r < 4; ++r) dst[r * D] = s[p][r];
@@ -793,7 +852,13 @@ extern "C" int npn_deltanet_chunked_prefill(const float* state, const float* que
   hipLaunchKernelGGL(dn_chunk_prep_kernel, dim3(std::min(items, kPrepGrid)), dim3(256), 0, st,
                      PrepArgs{query, key, g, beta, ws, S, nch, items});
   const int groups = (v_heads + 7) / 8;
-  hipLaunchKernelGGL(dn_chunk_scan_kernel, dim3(groups * 8 * NCB), dim3(kScanThreads), 0, st,
-                     ScanArgs{state, query, key, value, ws, out, new_state, S, nch, v_heads});
+  const ScanArgs sa{state, query, key, value, ws, out, new_state, S, nch, v_heads};
+  // 16-column blocks while they all run at once, one workgroup per CU (8 per head, every 8th
+  // head on the same XCD of 32 CUs); from 33 heads they would queue for the CUs and the 32-column
+  // form's fewer bytes per column count
+  if (groups <= 4)
+    hipLaunchKernelGGL(dn_chunk_scan_kernel<1>, dim3(groups * 64), dim3(kScanThreads), 0, st, sa);
+  else
+    hipLaunchKernelGGL(dn_chunk_scan_kernel<2>, dim3(groups * 32), dim3(kScanThreads), 0, st, sa);
   return npn_launch_status();
 }

@@ -55,6 +55,18 @@ def _run(ops, args, C):
     return out.cpu().numpy(), ns.cpu().numpy()
 
 
+@pytest.mark.parametrize("S", [1, 63, 64, 193])
+def test_column_block_widths_agree(ops, S):
+    """33 heads run in 32-column blocks, up to 32 in 16-column blocks; a head's results are the
+    same bits in both (the blocks' columns are independent and summed alike)."""
+    Hv = 33
+    args = _inputs(Hv, S, seed=S)
+    out, ns = _run(ops, args, 64)
+    for n in (1, 9, 32):
+        o, s = _run(ops, [a[:a.shape[0] // Hv * n] for a in args], 64)
+        assert np.array_equal(o, out[:n * S]) and np.array_equal(s, ns[:n * 128])
+
+
 @pytest.mark.parametrize("Hv,S,C,seed", [(12, 64, 64, 0), (12, 200, 16, 1), (48, 130, 64, 2),
                                          (4, 1, 64, 3), (3, 1000, 64, 4), (2, 63, 16, 5)])
 def test_chunked_prefill_matches_oracle(ops, Hv, S, C, seed):
