@@ -14,7 +14,7 @@
 //     and the RoPE rows come straight from the position table.
 //  2. attn: split-KV over a balanced partition. The (b, kv head) pairs' 32-key steps
 //     are laid end to end (prefix sums from a one-block plan kernel) and cut into
-//     W = min(kAttnWG, S / 16) equal ranges (S steps in all), one per workgroup of the
+//     W = attn_wgs(S, pairs) equal ranges (S steps in all), one per workgroup of the
 //     kAttnWG launched (the rest exit at once), so every workgroup streams the same
 //     number of K/V bytes whatever the kv_len spread; a range may cover the end of one
 //     pair and the start of the next. One wave per 16-row tile of the R rows; each
@@ -264,19 +264,28 @@ __device__ __forceinline__ int pair_kend(const int32_t* kv_len, int b, int T, in
   return L + T < s_max ? L + T : s_max;
 }
 
-// Workgroups that take part for S steps in all: kAttnWG, or fewer when that would leave a
-// workgroup under kMinSteps steps (small batches), so a workgroup's fixed costs (its q' rows,
-// its partial rows, the ring's fill) stay small against its key stream and a pair's
-// partials stay few for the merge.
-constexpr int kMinSteps = 16;
-__device__ __forceinline__ int attn_wgs(int S) {
-  const int w = S / kMinSteps;
-  return w < 1 ? 1 : (w > kAttnWG ? kAttnWG : w);
+// Workgroups that take part for S steps of P pairs in all: kAttnWG, or fewer for small batches,
+// where two chains set the time, a workgroup's S / W steps (about 1.4 us each) and the merge's
+// W / P segments of a pair (about 0.3 us each). Their sum is least at W = sqrt(4.7 S P); between
+// one and two workgroups per CU that is one per CU (277 instead of 256 measured 54.0 against
+// 47.9 us), and whole workgroups per pair where the lengths are equal. At least two steps each:
+// a workgroup has its q' rows to read and its ring to fill. Measured (24 q / 4 kv heads, T = 8,
+// calls in a graph) against a fixed 16 steps a workgroup, the rule before: B = 1, 64 keys 37.4 ->
+// 16.2 us, 2048 keys 33.0 -> 21.4, 8192 keys 35.3 -> 29.6, 18432 keys 41.1 -> 38.8; B = 3, 700
+// keys 37.0 -> 20.8; B = 8, 4096 keys 52.7 -> 46.3; B = 2, 32000 keys 78.5 -> 72.9.
+constexpr int kMinSteps = 2;
+constexpr int kAttnCU = 256;
+__device__ __forceinline__ int attn_wgs(int S, int P) {
+  int w = (int)fminf(sqrtf(4.7f * (float)S * (float)P), (float)kAttnWG);
+  if (w < kAttnWG) w = min(w, kAttnCU);
+  w = min(w, S / kMinSteps);
+  if (w < kAttnWG && w > P) w -= w % P;
+  return w < 1 ? 1 : w;
 }
 
-// Workgroup w's step range is [w * S / W, (w + 1) * S / W), W = attn_wgs(S).
-__device__ __forceinline__ int wg_first_step(int w, int S) {
-  return (int)((int64_t)w * S / attn_wgs(S));
+// Workgroup w's step range of W workgroups is [w * S / W, (w + 1) * S / W).
+__device__ __forceinline__ int wg_first_step(int w, int S, int W) {
+  return (int)((int64_t)w * S / W);
 }
 
 // Largest p in [0, P) with pstart[p] <= x (pstart is strictly increasing, pstart[0] = 0):
@@ -324,9 +333,10 @@ __global__ __launch_bounds__(NRT * 64, NST <= 2 ? 2 : 1) void gqa_attn_kernel(At
   constexpr int DPW = (KS + NRT - 1) / NRT;  // DMA instructions per wave per step
   const int wg = blockIdx.x;
   const int S = a.pstart[a.npairs];
-  if (wg >= attn_wgs(S)) return;
-  int x = wg_first_step(wg, S);
-  const int x_end = wg_first_step(wg + 1, S);
+  const int W = attn_wgs(S, a.npairs);
+  if (wg >= W) return;
+  int x = wg_first_step(wg, S, W);
+  const int x_end = wg_first_step(wg + 1, S, W);
   if (x >= x_end) return;
 
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -545,7 +555,7 @@ __global__ __launch_bounds__(NRT * 64, NST <= 2 ? 2 : 1) void gqa_attn_kernel(At
 // 3. merge a pair's segment partials, apply sigmoid(gate), write bf16. One 256-thread block
 //    per (query row, pair); lane l of every wave owns output dims 4l..4l+3 (float4 partial
 //    reads). The workgroups that covered pair p are w(first step) .. w(last step), with
-//    w(x) = ((x + 1) * W - 1) / S, W = attn_wgs(S). Wave q merges segments q, q + 4, ... of
+//    w(x) = ((x + 1) * W - 1) / S, W = attn_wgs(S, pairs). Wave q merges segments q, q + 4, ... of
 //    the pair (loads issued four segments at a time), and wave 0 then merges the four
 //    waves' (m, l, O) in wave order: a small batch's pairs have tens of segments each, which
 //    one wave walking them in turn paid for in memory latency.
@@ -567,14 +577,14 @@ __global__ __launch_bounds__(256) void gqa_merge_kernel(MergeArgs a) {
   const int grp = a.Hq / a.Hkv;
   const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int S = a.pstart[a.npairs];
-  const int64_t W = attn_wgs(S);
+  const int64_t W = attn_wgs(S, a.npairs);
   const int x0 = a.pstart[pr], x1 = a.pstart[pr + 1] - 1;
   const int w0 = (int)(((int64_t)(x0 + 1) * W - 1) / S);
   const int w1 = (int)(((int64_t)(x1 + 1) * W - 1) / S);
   const size_t stride_ml = (size_t)a.R * 2, stride_o = (size_t)a.R * DH;
   const float* pml = a.part_ml + ((size_t)(w0 + pr) * a.R + r) * 2;
   const float* po = a.part_o + ((size_t)(w0 + pr) * a.R + r) * DH + 4 * lane;
-  auto live = [&](int w) { return w <= w1 && wg_first_step(w, S) < wg_first_step(w + 1, S); };
+  auto live = [&](int w) { return w <= w1 && wg_first_step(w, S, (int)W) < wg_first_step(w + 1, S, (int)W); };
   const int t = r / grp, qh = g * grp + (r - t * grp);
   const size_t oi = (((size_t)b * a.T + t) * a.Hq + qh) * DH + 4 * lane;
   // The gate is needed only by wave 0's output, after the merge: its load is issued first.
@@ -680,14 +690,14 @@ __global__ __launch_bounds__(256) void gqa_merge_rows_kernel(MergeArgs a) {
   const int pr = blockIdx.y;
   const int b = pr / a.Hkv, g = pr - b * a.Hkv;
   const int S = a.pstart[a.npairs];
-  const int64_t W = attn_wgs(S);
+  const int64_t W = attn_wgs(S, a.npairs);
   const int x0 = a.pstart[pr], x1 = a.pstart[pr + 1] - 1;
   const int w0 = (int)(((int64_t)(x0 + 1) * W - 1) / S);
   const int w1 = (int)(((int64_t)(x1 + 1) * W - 1) / S);
   const size_t stride_ml = (size_t)a.R * 2, stride_o = (size_t)a.R * DH;
   const float* pml = a.part_ml + ((size_t)(w0 + pr) * a.R + r) * 2;
   const float* po = a.part_o + ((size_t)(w0 + pr) * a.R + r) * DH + 4 * lane;
-  auto live = [&](int w) { return w <= w1 && wg_first_step(w, S) < wg_first_step(w + 1, S); };
+  auto live = [&](int w) { return w <= w1 && wg_first_step(w, S, (int)W) < wg_first_step(w + 1, S, (int)W); };
   const int t = r / grp, qh = g * grp + (r - t * grp);
   const size_t oi = (((size_t)b * a.T + t) * a.Hq + qh) * DH + 4 * lane;
   const uint2 gate_bits = *reinterpret_cast<const uint2*>(a.gate + oi);

@@ -95,6 +95,21 @@ def test_tail_verify_matches_oracle(ops, B, T, Hq, Hkv, kv_lens, s_max):
     assert_rel_close(_run_verify(ops, d), _oracle_verify(d), out_unit=BF16_U, name="tail_verify")
 
 
+@pytest.mark.parametrize("B,T,kv_lens", [
+    (1, 1, [0]),                  # one step in all: one workgroup for four pairs
+    (1, 8, [25]),                 # two steps a pair
+    (1, 8, [700]),                # whole workgroups per pair
+    (3, 5, [1, 3000, 40]),        # ragged: ranges over pair ends
+    (2, 8, [9000, 9000]),         # one workgroup per CU
+    (7, 2, [2000] * 6 + [31]),    # two per CU
+])
+def test_tail_verify_small_batch_splits(ops, B, T, kv_lens):
+    """The number of workgroups that a small batch's steps are cut into, at its lower end and
+    around 256 and 512 workgroups."""
+    d = gqa_verify_inputs(B, T, 24, 4, kv_lens, max(kv_lens) + T, seed=B + T)
+    assert_rel_close(_run_verify(ops, d), _oracle_verify(d), out_unit=BF16_U, name="tail_verify")
+
+
 def test_tail_verify_many_short_ragged_pairs(ops):
     """160 (sequence, kv head) pairs with 0..300 cached rows: more 32-key steps than
     attention workgroups, so workgroup ranges start and end inside pairs and one
