@@ -854,8 +854,8 @@ extern "C" int npn_deltanet_chunked_prefill(const float* state, const float* que
   const int groups = (v_heads + 7) / 8;
   const ScanArgs sa{state, query, key, value, ws, out, new_state, S, nch, v_heads};
   // 16-column blocks while they all run at once, one workgroup per CU (8 per head, every 8th
-  // head on the same XCD of 32 CUs); from 33 heads they would queue for the CUs and the 32-column
-  // form's fewer bytes per column count
+  // head on the same XCD of 32 CUs); beyond that they would take turns on the CUs, each with
+  // half the columns for the same q, k and record bytes
   if (groups <= 4)
     hipLaunchKernelGGL(dn_chunk_scan_kernel<1>, dim3(groups * 64), dim3(kScanThreads), 0, st, sa);
   else
