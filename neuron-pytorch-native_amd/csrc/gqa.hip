@@ -14,7 +14,7 @@
 //     and the RoPE rows come straight from the position table.
 //  2. attn: split-KV over a balanced partition. The (b, kv head) pairs' 32-key steps
 //     are laid end to end (prefix sums from a one-block plan kernel) and cut into
-//     W = attn_wgs(S, pairs) equal ranges (S steps in all), one per workgroup of the
+//     W equal ranges (S steps in all; W from the plan, attn_wgs), one per workgroup of the
 //     kAttnWG launched (the rest exit at once), so every workgroup streams the same
 //     number of K/V bytes whatever the kv_len spread; a range may cover the end of one
 //     pair and the start of the next. One wave per 16-row tile of the R rows; each
@@ -144,7 +144,7 @@ struct QPrepArgs {
   uint16_t* qhi;   // [B][Hkv][R][DH]
   uint16_t* qlo;
   const int32_t* kv_len;
-  int32_t* pstart;  // [P + 1]
+  int32_t* pstart;  // [P + 2]
   int B, T, Hq, Hkv, R, P, s_max;
   int qblocks;      // blocks 1..qblocks prepare q'; any blocks after them append the new
   AppendArgs app;   // K/V rows to the cache (app.key != nullptr), one wave per row
@@ -152,10 +152,50 @@ struct QPrepArgs {
 
 __device__ __forceinline__ int pair_kend(const int32_t* kv_len, int b, int T, int s_max);
 
+// Workgroups that take part for S steps of P pairs of `nrt` 16-row tiles (one wave each), `equal`
+// when all pairs have as many steps. Two chains set a small batch's time, a workgroup's S / W
+// steps (about 1.4 us each) and the merge's W / P segments of a pair (about 0.3 us each); their
+// sum is least at W = sqrt(4.7 S P). Below kAttnWG that is cut to one workgroup per CU (a few CUs
+// with two: 54.0 against 47.9 us for one sequence of 32768 keys), except that lone waves keep 16
+// steps each (nrt = 1, one sequence of 49152 keys: 256 workgroups 74 us, 384 69). From kAttnWG on
+// the chip is full, and the partial rows that every workgroup writes (R x 1 KB), which the model
+// leaves out, count: three waves a workgroup do better with one per CU, and ragged batches from
+// 14 steps per CU on with 16 steps each (two waves: where a pair has 128 steps to cut). With
+// equal lengths, whole workgroups per pair save every pair a second partial; more than 128
+// pairs don't divide one per CU. At least two steps each, since a workgroup has its q' rows to
+// read and its ring to fill.
+// Measured (24 q / 4 kv heads, calls in a graph, us) with 16 steps a workgroup always, with
+// min(sqrt(4.7 S P), kAttnWG) whatever nrt and the lengths, and with this rule:
+//   T = 8, 17 sequences of 1500 keys 44.9, 54.2, 44.6; 33 of 600 47.6, 51.5, 42.7; 8 of 4096
+//   55.7, 49.2, 46.4; two of 32000 79.9, 76.2, 69.8; one of 64 38, 17, 17;
+//   T = 7, 4 of 2892 to 12954 50.0, 56.2, 49.8; 6 of 1969 to 6688 47.0, 51.4, 44.6;
+//   T = 4, 17 of 1500 47.4, 49.0, 42.3; T = 3, 3 of 6158 to 21369 58.2, 60.1, 57.5;
+//   T = 1, 17 of 1500 52.1, 44.4, 38.5.
+// Over 232 batches it is 1.32 and 1.03 times as fast as the other two. The first is nowhere faster
+// by more than two runs differ (4 %), the second by up to 7 % on two ragged batches.
+constexpr int kMinSteps = 2;
+constexpr int kAttnCU = 256;
+__device__ __forceinline__ int attn_wgs(int S, int P, int nrt, bool equal) {
+  const int by16 = min(max(S / 16, 1), kAttnWG);
+  int w = (int)fminf(sqrtf(4.7f * (float)S * (float)P), (float)kAttnWG);
+  if (w < kAttnWG) {
+    w = min(w, kAttnCU);
+    if (nrt == 1) w = max(w, by16);
+  } else if (by16 == kAttnWG ||
+             (!equal && S >= 14 * kAttnCU && (nrt > 2 || (nrt == 2 && S >= 128 * P)))) {
+    return by16;
+  } else if (nrt > 2 && (!equal || P <= kAttnCU / 2)) {
+    w = kAttnCU;
+  }
+  w = min(w, S / kMinSteps);
+  if (equal && w > P) w -= w % P;
+  return w < 1 ? 1 : w;
+}
+
 // The plan: pstart[p] = sum of the steps of pairs before p (exclusive scan over one block of
-// 256 threads), pstart[P] = all steps.
+// 256 threads), pstart[P] = all steps, pstart[P + 1] = the workgroups that take part.
 __device__ void plan_block(const int32_t* kv_len, int32_t* pstart, int P, int Hkv, int T,
-                           int s_max) {
+                           int s_max, int nrt) {
   __shared__ int part[256];
   const int t = threadIdx.x;
   const int per = (P + 255) / 256;
@@ -170,17 +210,24 @@ __device__ void plan_block(const int32_t* kv_len, int32_t* pstart, int P, int Hk
     part[t] += v;
     __syncthreads();
   }
-  int run = part[t] - sum;
+  const int S = part[255];
+  int run = part[t] - sum, odd = 0;
   for (int p = p0; p < p1; ++p) {
+    const int n = (pair_kend(kv_len, p / Hkv, T, s_max) + KS - 1) / KS;
     pstart[p] = run;
-    run += (pair_kend(kv_len, p / Hkv, T, s_max) + KS - 1) / KS;
+    run += n;
+    odd |= (int64_t)n * P != S;
   }
-  if (t == 255) pstart[P] = part[255];
+  odd = __syncthreads_or(odd);
+  if (t == 0) {
+    pstart[P] = S;
+    pstart[P + 1] = attn_wgs(S, P, nrt, odd == 0);
+  }
 }
 
 __global__ __launch_bounds__(256) void gqa_qprep_kernel(QPrepArgs a) {
   if (blockIdx.x == 0) {
-    plan_block(a.kv_len, a.pstart, a.P, a.Hkv, a.T, a.s_max);
+    plan_block(a.kv_len, a.pstart, a.P, a.Hkv, a.T, a.s_max, a.R / 16);
     return;
   }
   if ((int)blockIdx.x > a.qblocks) {
@@ -252,7 +299,7 @@ struct AttnArgs {
   const uint16_t* cache_k;
   const uint16_t* cache_v;
   const int32_t* kv_len;
-  const int32_t* pstart;  // [P + 1] first step of each pair; pstart[P] = total steps
+  const int32_t* pstart;  // [P + 2] first step of each pair, total steps, workgroups
   float* part_o;          // [kAttnWG + P][R][DH]
   float* part_ml;         // [kAttnWG + P][R][2]
   int Hkv, s_max, T, grp, npairs;
@@ -262,25 +309,6 @@ struct AttnArgs {
 __device__ __forceinline__ int pair_kend(const int32_t* kv_len, int b, int T, int s_max) {
   const int L = kv_len[b] > 0 ? kv_len[b] : 0;
   return L + T < s_max ? L + T : s_max;
-}
-
-// Workgroups that take part for S steps of P pairs in all: kAttnWG, or fewer for small batches,
-// where two chains set the time, a workgroup's S / W steps (about 1.4 us each) and the merge's
-// W / P segments of a pair (about 0.3 us each). Their sum is least at W = sqrt(4.7 S P); between
-// one and two workgroups per CU that is one per CU (277 instead of 256 measured 54.0 against
-// 47.9 us), and whole workgroups per pair where the lengths are equal. At least two steps each:
-// a workgroup has its q' rows to read and its ring to fill. Measured (24 q / 4 kv heads, T = 8,
-// calls in a graph) against a fixed 16 steps a workgroup, the rule before: B = 1, 64 keys 37.4 ->
-// 16.2 us, 2048 keys 33.0 -> 21.4, 8192 keys 35.3 -> 29.6, 18432 keys 41.1 -> 38.8; B = 3, 700
-// keys 37.0 -> 20.8; B = 8, 4096 keys 52.7 -> 46.3; B = 2, 32000 keys 78.5 -> 72.9.
-constexpr int kMinSteps = 2;
-constexpr int kAttnCU = 256;
-__device__ __forceinline__ int attn_wgs(int S, int P) {
-  int w = (int)fminf(sqrtf(4.7f * (float)S * (float)P), (float)kAttnWG);
-  if (w < kAttnWG) w = min(w, kAttnCU);
-  w = min(w, S / kMinSteps);
-  if (w < kAttnWG && w > P) w -= w % P;
-  return w < 1 ? 1 : w;
 }
 
 // Workgroup w's step range of W workgroups is [w * S / W, (w + 1) * S / W).
@@ -333,7 +361,7 @@ __global__ __launch_bounds__(NRT * 64, NST <= 2 ? 2 : 1) void gqa_attn_kernel(At
   constexpr int DPW = (KS + NRT - 1) / NRT;  // DMA instructions per wave per step
   const int wg = blockIdx.x;
   const int S = a.pstart[a.npairs];
-  const int W = attn_wgs(S, a.npairs);
+  const int W = a.pstart[a.npairs + 1];
   if (wg >= W) return;
   int x = wg_first_step(wg, S, W);
   const int x_end = wg_first_step(wg + 1, S, W);
@@ -555,7 +583,7 @@ __global__ __launch_bounds__(NRT * 64, NST <= 2 ? 2 : 1) void gqa_attn_kernel(At
 // 3. merge a pair's segment partials, apply sigmoid(gate), write bf16. One 256-thread block
 //    per (query row, pair); lane l of every wave owns output dims 4l..4l+3 (float4 partial
 //    reads). The workgroups that covered pair p are w(first step) .. w(last step), with
-//    w(x) = ((x + 1) * W - 1) / S, W = attn_wgs(S, pairs). Wave q merges segments q, q + 4, ... of
+//    w(x) = ((x + 1) * W - 1) / S, W from the plan. Wave q merges segments q, q + 4, ... of
 //    the pair (loads issued four segments at a time), and wave 0 then merges the four
 //    waves' (m, l, O) in wave order: a small batch's pairs have tens of segments each, which
 //    one wave walking them in turn paid for in memory latency.
@@ -577,7 +605,7 @@ __global__ __launch_bounds__(256) void gqa_merge_kernel(MergeArgs a) {
   const int grp = a.Hq / a.Hkv;
   const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int S = a.pstart[a.npairs];
-  const int64_t W = attn_wgs(S, a.npairs);
+  const int64_t W = a.pstart[a.npairs + 1];
   const int x0 = a.pstart[pr], x1 = a.pstart[pr + 1] - 1;
   const int w0 = (int)(((int64_t)(x0 + 1) * W - 1) / S);
   const int w1 = (int)(((int64_t)(x1 + 1) * W - 1) / S);
@@ -690,7 +718,7 @@ __global__ __launch_bounds__(256) void gqa_merge_rows_kernel(MergeArgs a) {
   const int pr = blockIdx.y;
   const int b = pr / a.Hkv, g = pr - b * a.Hkv;
   const int S = a.pstart[a.npairs];
-  const int64_t W = attn_wgs(S, a.npairs);
+  const int64_t W = a.pstart[a.npairs + 1];
   const int x0 = a.pstart[pr], x1 = a.pstart[pr + 1] - 1;
   const int w0 = (int)(((int64_t)(x0 + 1) * W - 1) / S);
   const int w1 = (int)(((int64_t)(x1 + 1) * W - 1) / S);
@@ -1092,7 +1120,7 @@ VerifyPlan plan(int B, int T, int Hq, int Hkv) {
   p.q_bytes = up((size_t)p.P * p.R * DH * 2);
   p.po_bytes = up(slots * p.R * DH * 4);
   p.pml_bytes = up(slots * p.R * 2 * 4);
-  p.ps_bytes = up((size_t)(p.P + 1) * 4);
+  p.ps_bytes = up((size_t)(p.P + 2) * 4);
   p.total = 2 * p.q_bytes + p.po_bytes + p.pml_bytes + p.ps_bytes;
   return p;
 }

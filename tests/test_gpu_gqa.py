@@ -96,18 +96,68 @@ def test_tail_verify_matches_oracle(ops, B, T, Hq, Hkv, kv_lens, s_max):
 
 
 @pytest.mark.parametrize("B,T,kv_lens", [
-    (1, 1, [0]),                  # one step in all: one workgroup for four pairs
+    (1, 1, [0]),                  # one step a pair: two workgroups for four pairs
     (1, 8, [25]),                 # two steps a pair
     (1, 8, [700]),                # whole workgroups per pair
     (3, 5, [1, 3000, 40]),        # ragged: ranges over pair ends
     (2, 8, [9000, 9000]),         # one workgroup per CU
-    (7, 2, [2000] * 6 + [31]),    # two per CU
+    (7, 2, [2000] * 6 + [31]),    # the same with one wave a workgroup
+    (7, 2, [3000] * 6 + [31]),    # two per CU
 ])
 def test_tail_verify_small_batch_splits(ops, B, T, kv_lens):
     """The number of workgroups that a small batch's steps are cut into, at its lower end and
     around 256 and 512 workgroups."""
     d = gqa_verify_inputs(B, T, 24, 4, kv_lens, max(kv_lens) + T, seed=B + T)
     assert_rel_close(_run_verify(ops, d), _oracle_verify(d), out_unit=BF16_U, name="tail_verify")
+
+
+@pytest.mark.parametrize("T,kv_lens,segments", [
+    (8, [64], 4),                          # two steps a workgroup, whole workgroups per pair
+    (1, [0], 4),                           # two workgroups of two steps, each of two pairs
+    (8, [1500] * 17, 204),                 # three waves a workgroup, up to 128 pairs: one per CU
+    (8, [600] * 33, 396),                  # more than 128 pairs: multiples of them up to 512
+    (4, [1500] * 17, 476),                 # two waves: up to two workgroups per CU
+    (4, [16000] * 2, 256),                 # few steps: one per CU
+    (2, [12000] * 3, 276),                 # one wave: 16 steps each rather than one per CU
+    (8, [1016] * 64, 512),                 # 16 steps for each of 512: all of them
+    (8, [738, 2600, 4464, 6327, 8191], 273),              # ragged: one per CU
+    (8, [179, 3461, 6743, 10025, 13307, 16590], 416),     # from 14 steps per CU: 16 each
+    (4, [1000, 9000, 20000], 267),         # few steps
+    (4, [866, 12476, 24086], 302),         # two waves, over 128 steps a pair: 16 steps each
+    (4, [700, 900, 1500, 1600] * 6, 594),  # fewer a pair: up to two workgroups per CU
+])
+def test_tail_verify_workgroups(ops, T, kv_lens, segments):
+    """The (workgroup, pair) segments that the attention kernel writes partials of, counted in
+    the workspace, and the first and last sequence against the oracle."""
+    from npn_native import call, query, stream_of
+    g = torch.Generator(device="cuda").manual_seed(sum(kv_lens))
+    r = lambda *n: torch.randn(*n, generator=g, device="cuda")  # noqa: E731
+    B, hq, hkv, s_max = len(kv_lens), 24, 4, max(kv_lens) + T
+    q, gate = (r(B, T, hq, 256).bfloat16() for _ in range(2))
+    k, v = (r(B, hkv, s_max, 256).bfloat16() for _ in range(2))
+    qn = r(256) * 0.1
+    cos, sin = (torch.from_numpy(t).cuda() for t in og.rope_cos_sin(
+        np.array(kv_lens)[:, None] + np.arange(T), theta=1e7))
+    kv_len = torch.tensor(kv_lens, dtype=torch.int32, device="cuda")
+    n_ws = query("npn_gqa_tail_verify_workspace_size", B, T, hq, hkv, s_max)
+    ws = torch.full((n_ws,), 255, dtype=torch.uint8, device="cuda")
+    out = torch.empty_like(q)
+    call("npn_gqa_tail_verify", q, gate, qn, cos, sin, k, v, kv_len, out, B, T, hq, hkv, s_max,
+         ws, n_ws, stream_of(q))
+    torch.cuda.synchronize()
+    # workspace: q' hi and lo [P][R][256] bf16, O [512 + P][R][256] f32, (m, l) [512 + P][R][2]
+    up = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    P, R = B * hkv, (T * hq // hkv + 15) // 16 * 16
+    off = 2 * up(P * R * 512) + up((512 + P) * R * 1024)
+    ml = ws[off:off + (512 + P) * R * 8].view(torch.int32).reshape(512 + P, R * 2)
+    assert (ml != -1).any(1).sum().item() == segments
+    for b in {0, B - 1}:
+        ref = og.gqa_tail_verify(*[bits(t[b:b + 1].cpu()) for t in (q, gate)], qn.cpu().numpy(),
+                                 *[t[b:b + 1].cpu().numpy() for t in (cos, sin)],
+                                 *[bits(t[b:b + 1].cpu()) for t in (k, v)],
+                                 kv_len[b:b + 1].cpu().numpy())
+        assert_rel_close(out[b:b + 1].float().cpu().double().numpy(), ref, out_unit=BF16_U,
+                         name=f"sequence {b}")
 
 
 def test_tail_verify_many_short_ragged_pairs(ops):
