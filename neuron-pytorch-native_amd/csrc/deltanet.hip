@@ -461,16 +461,23 @@ extern "C" int npn_deltanet_full_batched(const float* state, const uint16_t* mix
                                          uint16_t* new_conv_state, uint16_t* out, int B,
                                          int k_heads, int v_heads, void* stream) {
   NPN_REQUIRE(new_conv_state != nullptr, NPN_ERR_NULL);
-  const size_t n = B > 0 && k_heads > 0 && v_heads > 0
-                       ? (size_t)B * (2 * (size_t)k_heads + v_heads) * D
-                       : 0;
+  const size_t qkv = k_heads > 0 && v_heads > 0 ? (2 * (size_t)k_heads + v_heads) * D : 0;
+  const size_t hv = v_heads > 0 ? v_heads : 0, b = B > 0 ? B : 0, n = b * qkv;
   // The window shift goes with the verify launch: as a graph node of its own it cost 1.6 us
   // (calls in one graph, 4/12 heads: B = 1 7.1 -> 5.5 us, B = 8 7.6 -> 5.9, B = 64 18.7 -> 17.7;
-  // 16/48 heads: B = 1 7.4 -> 5.7, B = 8 12.7 -> 11.2). A caller's window that overlaps its input keeps the second launch: a group's
-  // heads all read the q and k windows that its first head would overwrite.
-  const uintptr_t c0 = reinterpret_cast<uintptr_t>(conv_state);
-  const uintptr_t n0 = reinterpret_cast<uintptr_t>(new_conv_state);
-  const bool overlap = n0 < c0 + 6 * n && c0 < n0 + 6 * n;
+  // 16/48 heads: B = 1 7.4 -> 5.7, B = 8 12.7 -> 11.2). A new window over any of the step's inputs
+  // keeps the second launch: a group's heads all read the q and k windows that its first head
+  // would overwrite, and workgroups that start late the rest.
+  auto over = [&](const void* in, size_t bytes) {
+    const uintptr_t i0 = reinterpret_cast<uintptr_t>(in);
+    const uintptr_t n0 = reinterpret_cast<uintptr_t>(new_conv_state);
+    return n0 < i0 + bytes && i0 < n0 + 6 * n;
+  };
+  const bool overlap = over(state, 4 * b * hv * D * D) || over(mixed_qkv, 2 * n) ||
+                       over(conv_state, 6 * n) || over(conv_weight, 16 * qkv) ||
+                       over(conv_bias, 4 * qkv) || over(a_out, 4 * b * hv) ||
+                       over(b_out, 4 * b * hv) || over(z, 2 * b * hv * D) ||
+                       over(A_log, 4 * hv) || over(dt_bias, 4 * hv) || over(norm_weight, 4 * D);
   const int st = verify_checked(state, nullptr, 0, mixed_qkv, conv_state, conv_weight, conv_bias,
                                 a_out, b_out, z, A_log, dt_bias, norm_weight, new_state, out,
                                 overlap ? nullptr : new_conv_state, B, 1, k_heads, v_heads,

@@ -113,6 +113,27 @@ def test_token_step_shifts_conv_window(ops, B, Hk, Hv, overlapping):
     assert torch.equal(state, ckpt) and torch.equal(bits_t(out), bits_t(vout))
 
 
+@pytest.mark.parametrize("name", ["state", "conv_weight", "a_out", "z", "norm_weight"])
+def test_window_over_a_step_input(ops, name):
+    """A new window written over an input that the token step alone reads: the step has read it
+    by then, so state and output are those of separate buffers."""
+    from npn_native import call, stream_of
+    B, Hk, Hv = 5, 16, 48
+    f = deltanet_flat_device(deltanet_inputs(B, 1, Hk, Hv, seed=7))
+    want = ops.deltanet.full_batched(*f.values())
+    raw = f[name].contiguous().view(torch.uint8).reshape(-1)
+    buf = torch.zeros(max(raw.numel(), B * (2 * Hk + Hv) * 128 * 6), dtype=torch.uint8,
+                      device="cuda")
+    buf[:raw.numel()] = raw
+    f[name] = buf[:raw.numel()].view(f[name].dtype).reshape(f[name].shape)
+    conv = buf[:want[1].numel() * 2].view(torch.bfloat16).reshape(want[1].shape)
+    state, out = torch.empty_like(want[0]), torch.empty_like(want[2])
+    call("npn_deltanet_full_batched", *f.values(), state, conv, out, B, Hk, Hv, stream_of(state))
+    torch.cuda.synchronize()
+    for got, ref in zip((state, conv, out), want):
+        assert torch.equal(got.view(torch.uint8), ref.view(torch.uint8))
+
+
 def test_rollback_copy_and_index(ops):
     """Copy rollback == ckpt[b, a_b]; conv window bit-exact; index-based next verify ==
     verify from the copied state (no copy needed)."""
