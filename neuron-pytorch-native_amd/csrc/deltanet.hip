@@ -463,11 +463,15 @@ extern "C" int npn_deltanet_full_batched(const float* state, const uint16_t* mix
   NPN_REQUIRE(new_conv_state != nullptr, NPN_ERR_NULL);
   const size_t qkv = k_heads > 0 && v_heads > 0 ? (2 * (size_t)k_heads + v_heads) * D : 0;
   const size_t hv = v_heads > 0 ? v_heads : 0, b = B > 0 ? B : 0, n = b * qkv;
-  // The window shift goes with the verify launch: as a graph node of its own it cost 1.6 us
-  // (calls in one graph, 4/12 heads: B = 1 7.1 -> 5.5 us, B = 8 7.6 -> 5.9, B = 64 18.7 -> 17.7;
-  // 16/48 heads: B = 1 7.4 -> 5.7, B = 8 12.7 -> 11.2). A new window over any of the step's inputs
-  // keeps the second launch: a group's heads all read the q and k windows that its first head
-  // would overwrite, and workgroups that start late the rest.
+  // The window shift goes with the verify launch while that is small: as a graph node of its own
+  // it cost 1.6 us (calls in one graph, own launch against this, 4/12 heads: B = 1 7.1, 5.5 us,
+  // B = 8 7.6, 5.9, B = 64 20.0, 19.0; 16/48 heads: B = 1 7.4, 5.7, B = 8 13.4, 11.4, B = 16
+  // 19.9, 19.0). In more workgroups than run at once (three per CU with 512 threads, 768 heads)
+  // its scattered 2-byte stores cost more than the launch: B = 20 24.8, 24.7; B = 24 29.4, 30.3;
+  // B = 48 63.6, 66.7; B = 64 83.9, 86.9. A new window over any of the step's inputs has its own
+  // launch too: a group's heads all read the q and k windows that its first head would
+  // overwrite, and workgroups that start late the rest.
+  const bool small = b * hv <= 768;
   auto over = [&](const void* in, size_t bytes) {
     const uintptr_t i0 = reinterpret_cast<uintptr_t>(in);
     const uintptr_t n0 = reinterpret_cast<uintptr_t>(new_conv_state);
@@ -480,9 +484,9 @@ extern "C" int npn_deltanet_full_batched(const float* state, const uint16_t* mix
                        over(A_log, 4 * hv) || over(dt_bias, 4 * hv) || over(norm_weight, 4 * D);
   const int st = verify_checked(state, nullptr, 0, mixed_qkv, conv_state, conv_weight, conv_bias,
                                 a_out, b_out, z, A_log, dt_bias, norm_weight, new_state, out,
-                                overlap ? nullptr : new_conv_state, B, 1, k_heads, v_heads,
-                                stream);
-  if (st != NPN_OK || !overlap) return st;
+                                small && !overlap ? new_conv_state : nullptr, B, 1, k_heads,
+                                v_heads, stream);
+  if (st != NPN_OK || (small && !overlap)) return st;
   hipLaunchKernelGGL(dn_conv_window_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), conv_state, mixed_qkv, nullptr,
                      new_conv_state, B, 1, (2 * k_heads + v_heads) * D);

@@ -7,6 +7,9 @@ and copy-based rollback, a B=32 full-size run checked on sampled sequences, and 
 column-split launch of small batches against the unsplit one, bit for bit.
 Bar: 2e-3 relative (tests/_util.py); conv windows are data movement and must be bit-exact.
 """
+import ctypes
+import os
+
 import numpy as np
 import pytest
 import torch
@@ -89,7 +92,8 @@ def test_full_batched_reference_shapes(ops, B):
 @pytest.mark.parametrize("B,Hk,Hv,overlapping", [
     (1, 16, 48, False),   # four workgroups per head store a share each
     (2, 3, 3, False),     # every head is its group's first
-    (33, 16, 48, False),  # two row parts
+    (16, 16, 48, False),  # the most heads that shift in the step's launch
+    (33, 16, 48, False),  # two row parts, a launch of its own
     (2, 4, 12, True),     # window shifted in place: a launch of its own
 ])
 def test_token_step_shifts_conv_window(ops, B, Hk, Hv, overlapping):
@@ -111,6 +115,22 @@ def test_token_step_shifts_conv_window(ops, B, Hk, Hv, overlapping):
     torch.cuda.synchronize()
     assert torch.equal(bits_t(conv), bits_t(want))
     assert torch.equal(state, ckpt) and torch.equal(bits_t(out), bits_t(vout))
+
+
+@pytest.mark.parametrize("B,Hk,Hv,launches", [(1, 16, 48, 1), (16, 16, 48, 1), (64, 4, 12, 1),
+                                              (17, 16, 48, 2), (65, 4, 12, 2)])
+def test_window_shift_launches(ops, B, Hk, Hv, launches):
+    """One launch while every head's workgroup runs at once (768 heads), two for more: there the
+    window's stores lengthen the step by more than a launch."""
+    f = deltanet_flat_device(deltanet_inputs(B, 1, Hk, Hv, seed=3))
+    ops.deltanet.full_batched(*f.values())
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        ops.deltanet.full_batched(*f.values())
+    hip = ctypes.CDLL(os.path.join(os.path.dirname(torch.__file__), "lib", "libamdhip64.so"))
+    n = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    assert n.value == launches
 
 
 @pytest.mark.parametrize("name", ["state", "conv_weight", "a_out", "z", "norm_weight"])
