@@ -1483,17 +1483,30 @@ void plan_wide128(int M, GemmPlan& p) {
 // empty or tiled 16 columns at a time: M = 4096 17408 x 5120 1600 -> 583 us, M = 700 5120 x
 // 16512 191 -> 112, M = 2048 5120 x 8704 282 -> 171, M = 2048 5120 x 34816 689 -> 601. Split-K
 // partials stay under 64 MB (they are written and read back through the memory-side cache).
+//
+// The 256-row kernel's groups of one row pass are dealt to the 8 XCDs in equal runs, so a number
+// that 8 doesn't divide fills some XCDs before others: 19 groups x 12 passes put 36 workgroups on
+// six XCDs of 32 CUs, and take two rounds though they are 228 (M = 3000, 5120 x 3584: 201 us,
+// with 240 workgroups of 128 rows 118). Up to 512 rows a split plan of the rule before stays
+// unless the model gives another 8 %: there it is no nearer than that (M = 385 to 512, 5120 x
+// 8704 with SwiGLU in two splits 58.1 to 61.6 us, unsplit 60.7 to 62.2, modelled 1 to 7 % faster).
 void plan_rows(int M, int K, int N, GemmPlan& p) {
   const int units = N / 16;
-  double best = 1e30;
-  auto offer = [&](bool rows128, int nh, bool odd, int per, int s) {
+  auto model = [&](bool rows128, int per, int s) {
     const int groups = (units + per - 1) / per;
-    const int rtiles = rows128 ? (M + 127) / 128 : (M + 255) / 256;
-    const long wgs = (long)groups * rtiles * s;
+    const long wgs = rows128 ? (long)groups * ((M + 127) / 128) * s
+                             : (long)((groups * s + 7) / 8 * 8) * ((M + 255) / 256);
     const int chunks = (K / KC + s - 1) / s;
     const double step = rows128 ? 0.226 + 0.0422 * per : 0.333 + 0.0741 * per;
     double t = (double)((wgs + WIDE_WG - 1) / WIDE_WG) * (chunks * step + 1.75);
     if (s > 1) t += 2.0 * s * M * N * 4 / 4.9e6 + 2.0;
+    return t;
+  };
+  double best = 1e30;
+  if (M <= 512 && p.split_k > 1)
+    best = model(p.rows128, p.rows128 ? 2 * p.h128 : 2 * p.ntm, p.split_k) / 1.08;
+  auto offer = [&](bool rows128, int nh, bool odd, int per, int s) {
+    const double t = model(rows128, per, s);
     if (t >= best) return;
     best = t;
     p.wide = true;
@@ -1502,7 +1515,7 @@ void plan_rows(int M, int K, int N, GemmPlan& p) {
     p.ntm = nh;
     p.h128 = rows128 ? per / 2 : 0;
     p.units = units;
-    p.groups = groups;
+    p.groups = (units + per - 1) / per;
     p.split_k = s;
   };
   for (int s = 1; s <= 8 && K / KC >= 2 * s; s *= 2) {

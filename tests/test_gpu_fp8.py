@@ -191,7 +191,11 @@ def test_rows128_plans(ops, M, K, N, S, U):
 @pytest.mark.parametrize("M,K,N,plan", [
     (385, 128, 34816, (3, 1, 18)), (4096, 128, 64, (3, 1, 4)), (4095, 128, 5120, (3, 1, 20)),
     (1025, 192, 8704, (3, 1, 20)), (700, 128, 16512, (2, 1, 7)), (2300, 128, 34816, (2, 1, 7)),
-    (513, 17408, 640, (3, 8, 8)), (770, 17408, 1344, (3, 4, 10)), (1200, 17408, 5120, (2, 2, 7))])
+    (513, 17408, 640, (3, 8, 8)), (770, 17408, 1344, (3, 4, 10)), (1200, 17408, 5120, (2, 2, 7)),
+    # 27, 23 and 19 groups of a row pass leave the XCDs uneven, so 256-row tiles would take two rounds
+    (2177, 128, 5120, (3, 1, 24)), (2561, 128, 5120, (3, 1, 14)), (3000, 128, 3584, (3, 1, 24)),
+    # up to 512 rows the one-pass rule's split stays where the model has nothing clear against it
+    (400, 5120, 8704, (3, 2, 18)), (512, 6144, 5120, (3, 4, 20))])
 def test_many_row_plans(ops, M, K, N, plan):
     """More than 256 rows: both wide kernels in one and several rounds of workgroups, with and
     without split-K, partial row tiles and column groups. Unsplit plans equal the 256-row
