@@ -1473,34 +1473,38 @@ void plan_wide128(int M, GemmPlan& p) {
   }
 }
 
+// Modelled time in us of a wide kernel (128- or 256-row tiles, `per` units of 16 columns and
+// `groups` workgroups per row tile, split-K factor s): rounds of 256 workgroups x (64-k chunks x
+// (a + b x per) + e) + partial traffic. The constants are a least-squares fit to 4,600 timings on
+// MI355X (seven projection shapes, 64 < M <= 3584, weights rotated through 400 MB, 5 % rms).
+// The 256-row kernel's groups of one row pass are dealt to the 8 XCDs in equal runs, so a number
+// that 8 doesn't divide fills some XCDs before others: 19 groups x 12 passes put 36 workgroups on
+// six XCDs of 32 CUs, and take two rounds though they are 228 (M = 3000, 5120 x 3584: 201 us,
+// with 240 workgroups of 128 rows 118).
+double wide_us(int M, int K, int N, bool rows128, int per, int groups, int s) {
+  const long wgs = rows128 ? (long)groups * ((M + 127) / 128) * s
+                           : (long)((groups * s + 7) / 8 * 8) * ((M + 255) / 256);
+  const int chunks = (K / KC + s - 1) / s;
+  const double step = rows128 ? 0.226 + 0.0422 * per : 0.333 + 0.0741 * per;
+  double t = (double)((wgs + WIDE_WG - 1) / WIDE_WG) * (chunks * step + 1.75);
+  if (s > 1) t += 2.0 * s * M * N * 4 / 4.9e6 + 2.0;
+  return t;
+}
+
 // Plan for more than 256 rows, where the grid usually takes several rounds of 256 workgroups:
-// the (kernel, tile width, split-K factor) with the least modelled time
-//   rounds x (64-k chunks x (a + b x units per workgroup) + e) + partial traffic
-// in us. The constants are a least-squares fit to 4,600 timings on MI355X (seven projection
-// shapes, 64 < M <= 3584, weights rotated through 400 MB, 5 % rms); its choice was within 1 %
-// of the best of all configurations on average. The rule before (each row pass planned as if
+// the (kernel, tile width, split-K factor) with the least modelled time (wide_us), within 1 % of
+// the best of all configurations on average. The rule before (each row pass planned as if
 // it were alone, 128-row tiles only when they fitted one round) left the last round nearly
 // empty or tiled 16 columns at a time: M = 4096 17408 x 5120 1600 -> 583 us, M = 700 5120 x
 // 16512 191 -> 112, M = 2048 5120 x 8704 282 -> 171, M = 2048 5120 x 34816 689 -> 601. Split-K
 // partials stay under 64 MB (they are written and read back through the memory-side cache).
-//
-// The 256-row kernel's groups of one row pass are dealt to the 8 XCDs in equal runs, so a number
-// that 8 doesn't divide fills some XCDs before others: 19 groups x 12 passes put 36 workgroups on
-// six XCDs of 32 CUs, and take two rounds though they are 228 (M = 3000, 5120 x 3584: 201 us,
-// with 240 workgroups of 128 rows 118). Up to 512 rows a split plan of the rule before stays
-// unless the model gives another 8 %: there it is no nearer than that (M = 385 to 512, 5120 x
-// 8704 with SwiGLU in two splits 58.1 to 61.6 us, unsplit 60.7 to 62.2, modelled 1 to 7 % faster).
+// Up to 512 rows a split plan of the rule before stays unless the model gives another 8 %: there
+// it is no nearer than that (M = 385 to 512, 5120 x 8704 with SwiGLU in two splits 58.1 to 61.6
+// us, unsplit 60.7 to 62.2, modelled 1 to 7 % faster).
 void plan_rows(int M, int K, int N, GemmPlan& p) {
   const int units = N / 16;
   auto model = [&](bool rows128, int per, int s) {
-    const int groups = (units + per - 1) / per;
-    const long wgs = rows128 ? (long)groups * ((M + 127) / 128) * s
-                             : (long)((groups * s + 7) / 8 * 8) * ((M + 255) / 256);
-    const int chunks = (K / KC + s - 1) / s;
-    const double step = rows128 ? 0.226 + 0.0422 * per : 0.333 + 0.0741 * per;
-    double t = (double)((wgs + WIDE_WG - 1) / WIDE_WG) * (chunks * step + 1.75);
-    if (s > 1) t += 2.0 * s * M * N * 4 / 4.9e6 + 2.0;
-    return t;
+    return wide_us(M, K, N, rows128, per, (units + per - 1) / per, s);
   };
   double best = 1e30;
   if (M <= 512 && p.split_k > 1)
@@ -1896,8 +1900,14 @@ bool fp8_matmul_stats_pass_cheaper(int M, int K, int N) {
   if (!fp8_matmul_chunk_stats_ok(M, K, N)) return true;
   const GemmPlan e = plan(M, K, N, true, 4);
   if (!e.wide) return false;
-  const int q_rounds = q.rows128 ? 1 : (q.groups + WIDE_WG - 1) / WIDE_WG;
-  return q_rounds < (e.groups + WIDE_WG - 1) / WIDE_WG;
+  // Measured at H = 5120 (us, epilogue against pass): whenever the plain plan is modelled faster
+  // the pass wins, M = 256, V = 248320 877, 773; M = 72, V = 32000 108, 76; M = 264, V = 16384 135,
+  // 94, V = 128256 802, 562; M = 512, V = 65536 456, 386; M = 1024, V = 92544 1227, 1125. At the same
+  // modelled time the two are even (M = 256, V = 32000 121, 123, V = 128256 443, 445).
+  auto us = [&](const GemmPlan& p) {
+    return wide_us(M, K, N, p.rows128, p.rows128 ? 2 * p.h128 : 2 * p.ntm, p.groups, 1);
+  };
+  return us(q) < us(e);
 }
 
 int fp8_matmul_unsplit(const uint16_t* x, const int8_t* w, const float* scale, uint16_t* out,

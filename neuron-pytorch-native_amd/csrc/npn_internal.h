@@ -18,9 +18,9 @@ int fp8_matmul_chunk_stats(const uint16_t* x, const int8_t* w, const float* scal
                            hipStream_t stream);
 
 // Whether the statistics are better computed by a pass over plain logits: true when the plain
-// GEMM's plan is the wide kernel without split-K and needs fewer rounds of workgroups than the
-// plan with the statistics epilogue (whose column groups must hold whole 64-column chunks,
-// 12 of the widest tile's 14 units), or when the epilogue plan is not available.
+// GEMM's plan is the wide kernel without split-K and is modelled faster than the plan with the
+// statistics epilogue (256-row tiles whose column groups hold whole 64-column chunks, 12 of the
+// widest tile's 14 units), or when the epilogue plan is not available.
 bool fp8_matmul_stats_pass_cheaper(int M, int K, int N);
 // out [M, N] = npn_fp8_matmul's output, for shapes whose plan has no split-K (no workspace);
 // NPN_ERR_SHAPE otherwise.

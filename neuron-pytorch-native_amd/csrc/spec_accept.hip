@@ -1366,10 +1366,10 @@ extern "C" int npn_argmax_parts(const void* parts, int nparts, int64_t* ids, flo
 }
 
 // ---- rejection sampling straight from the LM head --------------------------------------------
-// The LM head's GEMM writes the target logits in bf16 and, in its epilogue, the contract's
-// chunk statistics of every target row, so the target rows are never read back in full: the
-// statistics pass covers only the draft rows, and the sampling kernel re-reads only each
-// sequence's sampling row. The decisions equal npn_accept_rejection's on the same logits cast
+// The LM head's GEMM writes the target logits in bf16. Either its epilogue also writes the
+// contract's chunk statistics of every target row, so that the statistics pass covers only the
+// draft rows and the sampling kernel re-reads only each sequence's sampling row, or, where the
+// plain GEMM is the faster one by more, the pass reads the target rows too. The decisions equal npn_accept_rejection's on the same logits cast
 // to fp32 (every step of the contract sees the same values).
 namespace {
 

@@ -128,6 +128,22 @@ def gqa_verify_inputs(B, T, Hq, Hkv, kv_lens, s_max, seed, theta=1e7):
     )
 
 
+# ---- launches -------------------------------------------------------------------------
+
+def graph_launches(fn):
+    """Nodes of fn's launches captured as a HIP graph."""
+    import ctypes
+    import os
+    fn()
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        fn()
+    hip = ctypes.CDLL(os.path.join(os.path.dirname(torch.__file__), "lib", "libamdhip64.so"))
+    n = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
 # ---- FP8 ------------------------------------------------------------------------------
 
 def fp8_weights(N, K, seed, fp8_max=448.0, std=0.02):

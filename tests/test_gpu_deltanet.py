@@ -7,16 +7,13 @@ and copy-based rollback, a B=32 full-size run checked on sampled sequences, and 
 column-split launch of small batches against the unsplit one, bit for bit.
 Bar: 2e-3 relative (tests/_util.py); conv windows are data movement and must be bit-exact.
 """
-import ctypes
-import os
-
 import numpy as np
 import pytest
 import torch
 
 from oracle import deltanet as od
 from _util import (assert_rel_close, bits, deltanet_flat_device, deltanet_inputs,
-                   deltanet_oracle_args, BF16_U)
+                   deltanet_oracle_args, graph_launches, BF16_U)
 
 pytestmark = pytest.mark.gpu
 
@@ -123,14 +120,7 @@ def test_window_shift_launches(ops, B, Hk, Hv, launches):
     """One launch while every head's workgroup runs at once (768 heads), two for more: there the
     window's stores lengthen the step by more than a launch."""
     f = deltanet_flat_device(deltanet_inputs(B, 1, Hk, Hv, seed=3))
-    ops.deltanet.full_batched(*f.values())
-    g = torch.cuda.CUDAGraph(keep_graph=True)
-    with torch.cuda.graph(g):
-        ops.deltanet.full_batched(*f.values())
-    hip = ctypes.CDLL(os.path.join(os.path.dirname(torch.__file__), "lib", "libamdhip64.so"))
-    n = ctypes.c_size_t()
-    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
-    assert n.value == launches
+    assert graph_launches(lambda: ops.deltanet.full_batched(*f.values())) == launches
 
 
 @pytest.mark.parametrize("name", ["state", "conv_weight", "a_out", "z", "norm_weight"])

@@ -29,6 +29,7 @@ import numpy as np
 import pytest
 import torch
 
+from _util import graph_launches
 from oracle import fp8 as ofp8
 from oracle.numerics import bf16_bits_to_f32, f32_to_bf16_bits
 
@@ -203,13 +204,15 @@ def _zm(ws, R):
 
 
 @pytest.mark.parametrize("B,V,inv_t", [(32, 248320, 1.0), (4, 151936, 1.0 / 0.7),
-                                       (32, 16384, 1.0 / 0.7)])
+                                       (32, 16384, 1.0 / 0.7), (9, 16384, 1.0),
+                                       (33, 16384, 1.0), (33, 4096, 1.0 / 0.7)])
 def test_lm_head_chunk_stats_bit_exact(ops, B, V, inv_t):
     """The LM-head form's rows' Z and M against accept_rejection's and the oracle's. The shapes
     take both routes: the plain GEMM then a statistics pass (B = 32, V = 248320, where the
-    chunk-aligned epilogue plan would need an extra round of workgroups) and the statistics
-    written by the GEMM epilogue (the narrow kernel at B = 4; the wide kernel at B = 32,
-    V = 16384, where both plans fit one round)."""
+    chunk-aligned epilogue plan would need an extra round of workgroups; 128-row tiles at B = 9
+    and 33, V = 16384) and the statistics written by the GEMM epilogue (the narrow kernel at
+    B = 4; the wide kernel at B = 32, V = 16384, where both plans are the same, and in two row
+    passes at V = 4096, where the plain plan splits K)."""
     from oracle import accept as oa
     from npn_native import call, query, stream_of
     K, H = 7, 1024
@@ -219,7 +222,12 @@ def test_lm_head_chunk_stats_bit_exact(ops, B, V, inv_t):
     hid[1, 5] = float("inf")                     # rows of +-inf and NaN logits
     hid[T + 2, 7] = float("nan")
     w, sc = _gpu_weights(H, V, B + 5)
-    logits = ops.fp8.matmul(hid, w, sc).float().view(B, T, V).contiguous()
+    logits = ops.fp8.matmul(hid, w, sc)
+    if query("npn_fp8_matmul_split_k", B * T, H, V) > 1:  # the op never splits K
+        gmax = torch.empty((B * T, query("npn_fp8_matmul_argmax_groups", B * T, H, V)),
+                           device="cuda")
+        call("npn_fp8_matmul_rowmax", hid, w, sc, logits, gmax, B * T, H, V, stream_of(hid))
+    logits = logits.float().view(B, T, V).contiguous()
     draft = (0.8 * logits[:, :K].nan_to_num(0.0, 50.0, -50.0)
              + 0.6 * torch.randn(B, K, V, generator=g, device="cuda")).contiguous()
     ids = torch.randint(0, V, (B, K), generator=g, device="cuda")
@@ -252,3 +260,20 @@ def test_lm_head_chunk_stats_bit_exact(ops, B, V, inv_t):
         _, Z, M = oa.row_weights(row, inv_t)
         assert z_lm[r] == Z, f"row {r}"
         assert m_lm[r].view(np.uint32) == np.float32(M).view(np.uint32), f"row {r}"
+
+
+@pytest.mark.parametrize("B,V,launches", [
+    (4, 16384, 5), (9, 16384, 4), (32, 16384, 5), (32, 65536, 5), (33, 4096, 5), (33, 16384, 4),
+    (33, 65536, 4), (64, 16384, 4), (64, 32000, 4)])
+def test_lm_head_route(ops, B, V, launches):
+    """The statistics pass (GEMM, statistics, mass, pick: four launches) where the plain GEMM is
+    unsplit and its plan is the faster one over all its rounds, at up to 256 rows and above;
+    else the epilogue (draft statistics, GEMM, blocks, mass, pick: five)."""
+    K, H = 7, 1024
+    g = torch.Generator(device="cuda").manual_seed(B + V)
+    hid = torch.randn(B * (K + 1), H, generator=g, device="cuda").to(torch.bfloat16)
+    w, sc = _gpu_weights(H, V, B)
+    args = (hid, w, sc, torch.randn(B, K, V, generator=g, device="cuda"),
+            torch.randint(0, V, (B, K), generator=g, device="cuda"),
+            torch.rand(B, K, generator=g, device="cuda"), torch.rand(B, generator=g, device="cuda"))
+    assert graph_launches(lambda: ops.spec.accept_rejection_lm_head(*args)) == launches
