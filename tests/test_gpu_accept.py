@@ -91,6 +91,28 @@ def test_rejection_bit_exact(ops, B, K, V, seed, inv_t):
     assert np.array_equal(out, rout)
 
 
+@pytest.mark.parametrize("B,K,V,inv_t", [
+    (85, 1, 16389, 1.0), (85, 1, 16389, 0.7),    # 255 mass workgroups: runs of 8 entries
+    (128, 1, 16384, 0.7),                        # 256 of them
+    (86, 1, 16389, 1.0), (86, 1, 16389, 0.7),    # 258: runs of 32
+    (257, 1, 100, 1.4),                          # one block a row, less than a sub-chunk
+])
+def test_rejection_mass_forms(ops, B, K, V, inv_t):
+    """Both forms of the mass kernel beside the number of workgroups that divides them, with and
+    without a temperature, against the oracle; the first sequences alone, in the other form,
+    give the same."""
+    target, draft, ids, u, us = _rejection_inputs(B, K, V, B + V, rho=0.5)
+    acc, out = _rejection(ops, target, draft, ids, u, us, inv_t)
+    racc, rout = oa.accept_rejection(target.numpy(), draft.numpy(), ids.numpy(), u.numpy(),
+                                     us.numpy(), inv_t)
+    assert np.array_equal(acc, racc) and np.array_equal(out, rout)
+    assert 0 < acc.mean() < K
+    n = 40
+    acc1, out1 = _rejection(ops, target[:n].contiguous(), draft[:n].contiguous(), ids[:n], u[:n],
+                            us[:n], inv_t)
+    assert np.array_equal(acc1, acc[:n]) and np.array_equal(out1, out[:n])
+
+
 def test_rejection_equal_distributions_always_accept(ops):
     target, _, ids, u, us = _rejection_inputs(6, 5, 3000, 9)
     acc, out = _rejection(ops, target, target[:, :5].contiguous(), ids, u, us)

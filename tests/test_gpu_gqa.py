@@ -45,8 +45,8 @@ def test_tail_key_splits(ops, B, HQ, S):
     workgroup per sequence, with masked keys anywhere; the workspace-free C entry (always one
     split) beside it. Each score is an fp32 sum of 256 products of total size about |q'||k| / 16
     = 16, off by about sqrt(256) 2^-24 16 = 1.5e-5, and so is its weight relative to the others:
-    the bound is six times that. An infinite V entry in the last row, next to the rows that a
-    partial tile clamps to it, stays in its own column."""
+    the bound is six times that. An infinite V entry in the last row, beside the rows past S
+    that a partial tile reads as 0, stays in its own column."""
     from npn_native import call, stream_of
     g = torch.Generator().manual_seed(B + HQ + S)
     r = lambda *n: torch.randn(*n, generator=g)  # noqa: E731

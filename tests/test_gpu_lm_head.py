@@ -194,6 +194,27 @@ def test_accept_rejection_lm_head(ops, B, V, inv_t):
     assert 0 < acc_f.float().mean() < K  # neither all accepted nor all rejected
 
 
+@pytest.mark.parametrize("B,inv_t", [(85, 0.7), (86, 0.7), (86, 1.0)])
+def test_lm_head_mass_forms(ops, B, inv_t):
+    """bf16 target rows through both forms of the mass kernel (up to 256 workgroups, and more):
+    the decisions of accept_rejection on the same logits as fp32, which the oracle checks."""
+    K, H, V = 1, 512, 16448
+    g = torch.Generator(device="cuda").manual_seed(B)
+    hid = torch.randn(B * 2, H, generator=g, device="cuda").to(torch.bfloat16)
+    w, sc = _gpu_weights(H, V, B)
+    base = ops.fp8.matmul(hid, w, sc).float().view(B, 2, V)
+    draft = (0.5 * base[:, :K]
+             + 0.8 * torch.randn(B, K, V, generator=g, device="cuda")).contiguous()
+    ids = torch.multinomial(torch.softmax(draft * inv_t, -1).reshape(B * K, V), 1,
+                            generator=g).reshape(B, K)
+    u, us = (torch.rand(*n, generator=g, device="cuda") for n in ((B, K), (B,)))
+    acc, out, lg = ops.spec.accept_rejection_lm_head(hid, w, sc, draft, ids, u, us, inv_t)
+    acc_r, out_r = ops.spec.accept_rejection(lg.float().contiguous(), draft, ids, u, us, inv_t)
+    torch.cuda.synchronize()
+    assert torch.equal(acc, acc_r) and torch.equal(out, out_r)
+    assert 0 < acc.float().mean() < K
+
+
 def _zm(ws, R):
     """Every row's Z (unsigned 128-bit, low word first) and M from a rejection workspace."""
     off = (16 * R + 255) // 256 * 256
