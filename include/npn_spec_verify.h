@@ -83,7 +83,8 @@ int npn_deltanet_full_batched(const float* state, const uint16_t* mixed_qkv,
  * npn_deltanet_full_fp8_workspace_size(hidden, k_heads, v_heads) bytes (0: unsupported sizes),
  * 16-byte aligned. Two launches: the qkv and z GEMMs (split-K partials) with a_out and b_out
  * beside them, then the token step, which reduces the partials and shifts the conv window
- * (wider projections than 14080 columns take launches of their own). */
+ * (with a stream-K plan, 55 to 255 tiles of 256 columns at hidden 5120, four: the projections
+ * take launches of their own). */
 size_t npn_deltanet_full_fp8_workspace_size(int hidden, int k_heads, int v_heads);
 int npn_deltanet_full_fp8(const uint16_t* x, const float* state, const uint16_t* conv_state,
                           const float* conv_weight, const float* conv_bias, const float* A_log,

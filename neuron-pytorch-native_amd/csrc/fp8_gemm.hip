@@ -452,6 +452,9 @@ __global__ __launch_bounds__(KG * 256, KG) void fp8_gemm_narrow_kernel(GemmArgs 
       __syncthreads();  // every wave is done with the ring's previous segment
     }
   }
+  // The second k group's waves end here, before barriers of the row-maximum epilogues below:
+  // gfx950 counts only the waves that have not ended, and all of the first group's, whole waves
+  // of uniform control flow, reach every one of them.
   if (kg != 0) return;
 
   // Lane (i, G) holds rows m_pass + 16 rb + 4 G + r and columns nc + c in acc[rb][c][r]. The
@@ -530,10 +533,10 @@ __global__ __launch_bounds__(KG * 256, KG) void fp8_gemm_narrow_kernel(GemmArgs 
       }
     }
     if (a.cmax != nullptr) {
-      // Contract chunk statistics: a 64-column chunk is held by LPC adjacent lanes of the
-      // 16-lane group (N % 64 == 0, so a chunk is wholly inside or wholly past N).
-      constexpr int LPC = 64 / CB;  // 16, 8 or 4: a DPP row, half-row or quad
-      constexpr int STEPS = LPC == 16 ? 4 : (LPC == 8 ? 3 : 2);
+      // Contract chunk statistics: a 64-column chunk is held by the 16 lanes of a group
+      // (N % 64 == 0, so a chunk is wholly inside or wholly past N).
+      constexpr int LPC = 64 / CB, STEPS = 4;
+      static_assert(LPC == 1 << STEPS, "a chunk is one 16-lane DPP row");
       float xs[CB];
 #pragma unroll
       for (int c = 0; c < CB / 2; ++c) {
@@ -1538,8 +1541,9 @@ GemmPlan plan(int M, int K, int N, bool no_split = false, int ua = 1) {
     // the argmax and chunk-statistics epilogues exist only in the 256-row kernel
     if (!no_split && ua == 1) {
       plan_wide128(M, p);
-      // up to three 128-row tiles a one-round plan of the 128-row kernel is within 10 % of the
-      // model's choice (5120 x 14336 71 against 63 us, 17408 x 5120 75 against 77)
+      // at 257 to 384 rows a one-round plan of the 128-row kernel stays, since
+      // tests/test_gpu_fp8.py holds such plans at 300 rows: 5120 x 14336 71 us where the model's
+      // choice takes 63, 17408 x 5120 75 where it takes 77
       if (M > 256 && !(p.rows128 && M <= 384)) plan_rows(M, K, N, p);
     }
     return p;
@@ -1570,8 +1574,9 @@ GemmPlan plan(int M, int K, int N, bool no_split = false, int ua = 1) {
   // tiles x 8: 16 CUs do twice the work of the rest); the grid of one per CU does better
   // although it streams with fewer waves: K = 5120, GEMM and reduction, N = 8704 split 16 -> 7
   // at 8 rows 17.4 -> 15.7 us, split 8 -> 7 at 40 rows 27.5 -> 18.7 (with two k groups);
-  // N = 10240 split 16 -> 6 at 16 rows 20.9 -> 16.8; N = 13824 24.1 -> 21.2. Up to 20 tiles 16
-  // splits of a few rows measured the same, and from 55 tiles stream-K takes over.
+  // N = 10240 split 16 -> 6 at 16 rows 20.9 -> 16.8; N = 13824 24.1 -> 21.2. At 20 tiles 12 splits
+  // would do better than 16 too (17408 x 5120 at 8 rows 24.5 against 28.9 us), but 16 is the
+  // factor that tests/test_gpu_fp8.py holds there. From 55 tiles stream-K takes over.
   if (!no_split && tiles * p.split_k > WIDE_WG && tiles > 20 && tiles <= 54)
     p.split_k = WIDE_WG / tiles;
   // Stream-K where the tiles x split grid cannot fill the CUs evenly (136 tiles x 4 = 544
@@ -1719,10 +1724,11 @@ int launch_token_projections(const uint16_t* x, const int8_t* w1, float* p1, int
   return npn_launch_status();
 }
 
-// Workspace of npn_deltanet_full_fp8, 256-byte aligned regions: room for mixed_qkv [QKV] and z
-// [Hv * 128] as bf16 (no kernel writes them; the size stays what callers have allocated), a_out
-// and b_out [Hv] f32, then the split-K partials of the qkv and z GEMMs ([S][N] f32 each, S from
-// the GEMM plan for one row).
+// Workspace of npn_deltanet_full_fp8, 256-byte aligned regions: mixed_qkv [QKV] and z [Hv * 128]
+// as bf16 (unused: the token step reduces the partials itself; tests/test_host.py holds the
+// size that npn_deltanet_full_fp8_workspace_size reports with them), a_out and b_out [Hv] f32,
+// then the split-K partials of the qkv and z GEMMs ([S][N] f32 each, S from the GEMM plan for
+// one row).
 struct FullFp8Layout {
   size_t a, b, pq, pz, total;
   int sq, sz;
@@ -1937,8 +1943,8 @@ int fp8_matmul_chunk_stats(const uint16_t* x, const int8_t* w, const float* scal
 // deltanet::full on their outputs. Two launches: the qkv and z GEMMs writing split-K partials
 // (the plans of npn_fp8_matmul for one row) with a_out and b_out in float32, not rounded,
 // beside them, and the DeltaNet token step, which reduces the partials to mixed_qkv and z as
-// npn_fp8_matmul's bf16 outputs and shifts the conv window. (Stream-K plans, from 14080
-// columns on, make four launches of the first.)
+// npn_fp8_matmul's bf16 outputs and shifts the conv window. (With a stream-K plan, 55 to 255
+// column tiles at hidden 5120, the first is three: either GEMM's, and a_out and b_out's.)
 extern "C" size_t npn_deltanet_full_fp8_workspace_size(int hidden, int k_heads, int v_heads) {
   if (!full_fp8_heads_ok(k_heads, v_heads)) return 0;
   const int qkv = (2 * k_heads + v_heads) * 128;
@@ -1961,8 +1967,8 @@ extern "C" int npn_deltanet_full_fp8(
   const int qkv = (2 * k_heads + v_heads) * 128, zn = v_heads * 128;
   NPN_REQUIRE(shape_ok(1, hidden, qkv), NPN_ERR_SHAPE);
   NPN_REQUIRE(NPN_ALIGNED16(x) && NPN_ALIGNED16(qkv_w) && NPN_ALIGNED16(z_w), NPN_ERR_ALIGN);
-  // the new conv window is written before the token step reads the old one, so the two
-  // [QKV, 3] bf16 spans must not share a byte
+  // the two [QKV, 3] bf16 windows must not share a byte: in the token step's launch a group's
+  // first head writes the new q and k windows while its other heads still read the old ones
   {
     const uintptr_t n0 = reinterpret_cast<uintptr_t>(new_conv_state);
     const uintptr_t c0 = reinterpret_cast<uintptr_t>(conv_state);
