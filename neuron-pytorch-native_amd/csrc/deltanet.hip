@@ -104,8 +104,8 @@ __device__ __forceinline__ uint16_t part_value(const float* part, int S, int n,
 // blocks apart, so with heads % 8 == 0 they share an XCD (and its L2 copy of the state).
 // PARTS (one token of one sequence): mixed_qkv and z come as the projections' split-K partials,
 // which every workgroup reduces for its own head's channels. As a kernel of its own between the
-// GEMM and this one the reduction took 4.7 to 5.9 us (deltanet::full_fp8, 16/48 heads, graph
-// replays: 31.4 us with it, 28.1 without).
+// GEMM and this one the reduction took 5.7 us at least and 6.6 on average (deltanet::full_fp8,
+// 16/48 heads, 100 calls in a graph: 30.3 us a call with it, 24.7 without).
 template <int TMAX, int P, bool PARTS>
 __global__ __launch_bounds__(128 * P) void dn_verify_kernel(DnArgs a) {
   static_assert(!PARTS || TMAX == 1, "partials of one token");
